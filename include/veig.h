@@ -44,9 +44,8 @@ typedef enum {
 #define VEIG_WRITE_SCHUR 1u /* also store the Schur form T over A (zeros below the diagonal) */
 
 /* Largest orders.  VEIG_MAX_DIM: veig_zgeev (FP64), veig_host_eigensolver and
- * the stage entries (orders above 64, and above 32 at the stage entries, run
- * on one workgroup per matrix with the matrix in LDS: 96 x 97 complex doubles
- * fill the LDS of a CU).  VEIG_MAX_DIM_FAST: veig_zgeev_fp32,
+ * the stage entries (orders above 32 run on one workgroup per matrix with the
+ * matrix in LDS: 96 x 97 complex doubles fill the LDS of a CU).  VEIG_MAX_DIM_FAST: veig_zgeev_fp32,
  * veig_zgeev_mixed, the eigenvalues-only and roots entries.
  * VEIG_MAX_DIM_VARSIZE: veig_zgeev_varsize (larger orders get info = -1). */
 #define VEIG_MAX_DIM 96
@@ -69,10 +68,9 @@ const char *veig_version(void);
  * info (may be NULL): per matrix, the number of eigenvalues accepted after
  * `itmax` sweeps without a negligible subdiagonal (the reference caps at 30,
  * Toolbox.hpp:808, and reports nothing; itmax <= 0 selects 30).
- * A, E and V are separate arrays: at orders 9..64 the call passes the
+ * A, E and V are separate arrays: above order 8 the call passes the
  * Hessenberg reduction's compact form between its kernels through V and E,
- * which then receive the results; above 64, V holds Q and then the Schur
- * vectors on the way to the eigenvectors.
+ * which then receive the results.
  * ------------------------------------------------------------------------- */
 int veig_zgeev(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rA, double *iA,
                double *rE, double *iE, double *rV, double *iV, int32_t *info, int32_t itmax,

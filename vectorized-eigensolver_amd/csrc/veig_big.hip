@@ -1,490 +1,300 @@
-// Orders beyond the lane-group kernels: the fused eigendecomposition at
-// 64 < n <= VEIG_MAX_DIM and the stage entries at 32 < n <= VEIG_MAX_DIM.
+// FP64 orders 33..96: the fused eigendecomposition of whole batches and lists,
+// the stage entries, and the roots entry's Schur form.
 //
-// One workgroup of 256 threads per matrix (a persistent grid walks the
-// batch).  The matrix being reduced or iterated lives in LDS as a dense
-// n x (n+1) column-major tile (at n = 96: 146 KB, most of the LDS of a CU);
-// the unitary factor (Q, the Schur vectors, V) stays in global memory, in the
-// caller's output planes, each thread owning one of its rows.  The
-// arithmetic is that of the lane-group kernels (veig_device.hpp) spread over
-// threads instead of lanes of a group, with workgroup barriers where those
-// use wavefront fences:
-//   reduction   zgehrd (Toolbox.hpp:1315-1490), LAPACK zlarfg sign, Q
-//               accumulated forward (Q <- Q H_i) when wanted;
-//   Q alone     zunghr (Toolbox.hpp:1492-1659) as the same forward product;
-//   QR          zlahqr_schur (Toolbox.hpp:690-1031): the deflation test,
-//               shifts and 30-sweep cap of lahqr, the bulge chase of
-//               sweep_step (rows from the left, barrier, columns and Schur
-//               vectors from the right, barrier);
-//   eigenvectors ztrevc + backsubstitution (Toolbox.hpp:1133-1313, 31-136):
-//               thread k solves for eigenvector k in column k of the tile,
-//               then thread r forms row r of V = Z X in place.
-// These orders are for coverage of the reference's interface (its own
-// driver sweeps n = 10..79, zlahqr.cpp:206-249); the bulge chase is a chain
-// of barriers and runs far below the lane-group kernels' rate.
+// One matrix per workgroup, two kernels:
+//
+//   k_reduce<CAP, W>   the Hessenberg reduction on a dense LDS tile
+//                      (reduce_block); for the fused path its compact form
+//                      goes to the V and E planes, which serve as workspace;
+//                      for the stages also Q (hessenberg, zunghr).
+//   k_schur<SL, NT>    wavefront 0 runs the QR iteration on the banded tile
+//                      (lahqr_stream), the others hold the Schur vectors in
+//                      registers, NT lanes per row, and replay the recorded
+//                      sweeps (SchurRows); then the eigenvector solve and
+//                      V = Z X on the matrix cores.
+//
+// Segments: the row of a Schur vector is cut so that a lane's part fits the
+// registers of three wavefronts per SIMD: two segments of 24 or 32 columns up
+// to order 64, four of 20 or 24 above (wider rows, the same registers).  LDS
+// is allocated for the batch's order: 40 KB at n = 64 (four matrices per CU),
+// 76 KB at n = 88 (two).  Up to 24 columns the allocation is held to four
+// wavefronts per SIMD although that spills (order 48 x 8,192: 12.3 -> 11.5 ms,
+// order 79 x 3,328: 51 -> 34 ms, whose two workgroups of six wavefronts do not
+// share a CU at three), at 32 columns to three.
+//
+// Measured (both kernels; in brackets the kernels these replaced, whose bulge
+// chase went through LDS): order 64 x 65,536 194 ms (368), order 79 x 3,328
+// 38 ms (233: a workgroup barrier per half step and Z in global memory), the
+// stages hessenberg + zlahqr + ztrevc at order 40 x 2,048 3.2 ms (21).  What
+// bounds order 64 now is the chain wavefront's instruction issue: 7,700 steps
+// of 600 cycles and 230 sweeps of 2,400 more are 2.2 of the 2.3 ms that four
+// matrices take on a CU.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 #include <string>
 
-#include "veig_common.hpp"
+#include "veig_stream.hpp"
 
 using namespace veig;
 
 namespace {
 
-constexpr int kThreads = 256;
-
-// element (r, c) of a matrix held in global split planes
-struct GMat {
-  double *re, *im;
-  int64_t base, sr, sc;
-  __device__ __forceinline__ int64_t idx(int r, int c) const { return base + r * sr + c * sc; }
-  __device__ __forceinline__ cx<double> ld(int r, int c) const {
-    const int64_t i = idx(r, c);
-    return mk<double>(re[i], im[i]);
-  }
-  __device__ __forceinline__ void st(int r, int c, cx<double> v) const {
-    const int64_t i = idx(r, c);
-    re[i] = v.re;
-    im[i] = v.im;
-  }
-};
-
-// the LDS tile: H(r, c) at t[c * ld + r], and a vector of n entries after it
-struct Tile {
-  double2 *t;
-  double2 *v;
-  int n, ld;
-  __device__ __forceinline__ double2 *at(int r, int c) const { return t + c * ld + r; }
-};
-
-// workgroup-wide helpers (every thread calls them)
-struct Shared {
-  double part[kThreads / 64];
-  int flag;
-};
-
-__device__ __forceinline__ double block_sum(double x, Shared &sh) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-  const int w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) sh.part[w] = x;
-  __syncthreads();
-  double s = 0;
-#pragma unroll
-  for (int q = 0; q < kThreads / 64; ++q) s += sh.part[q];
-  __syncthreads();
-  return s;
-}
-
-// largest value of `k` over the threads with `pred` (0 if none)
-__device__ __forceinline__ int block_max_index(bool pred, int k, Shared &sh) {
-  if (threadIdx.x == 0) sh.flag = 0;
-  __syncthreads();
-  if (pred) atomicMax(&sh.flag, k);
-  __syncthreads();
-  const int r = sh.flag;
-  __syncthreads();
-  return r;
-}
-
-// ---------------------------------------------------------------------------
-// Hessenberg reduction of the tile (zgehrd with zlarfg's LAPACK sign and its
-// x = 0 guard).  keep: leave v(i+2:n) below the subdiagonal and tau(i) in
-// tau_out (zgehrd's compact form); else zeros there.  Q (if non-null rows):
-// Q <- Q H_i for each reflector, Q in global memory, thread r owning row r.
-// ---------------------------------------------------------------------------
-__device__ void reduce_tile(const Tile &T, Shared &sh, bool keep, const GMat *Q, double2 *tau_out) {
-  const int n = T.n, tid = threadIdx.x;
-  for (int i = 0; i + 1 < n; ++i) {
-    double part = 0;
-    for (int r = i + 2 + tid; r < n; r += kThreads) {
-      const double2 h = *T.at(r, i);
-      part += h.x * h.x + h.y * h.y;
-    }
-    const double xnorm2 = block_sum(part, sh);
-    const double2 al = *T.at(i + 1, i);
-    const cx<double> alpha = mk(al.x, al.y);
-    cx<double> tau = mk<double>(0, 0), scal = mk<double>(0, 0);
-    double beta = alpha.re;
-    if (!(xnorm2 == 0.0 && alpha.im == 0.0)) {
-      const double nrm = fsqrt(abs2(alpha) + xnorm2);
-      beta = alpha.re >= 0.0 ? -nrm : nrm;
-      const double ib = frcp(beta);
-      tau = mk((beta - alpha.re) * ib, -alpha.im * ib);
-      scal = inv(mk(alpha.re - beta, alpha.im));
-    }
-    // v(i+1) = 1, v(r) = H(r, i) scal below; v zero elsewhere
-    for (int r = tid; r < n; r += kThreads) {
-      cx<double> vr = mk<double>(0, 0);
-      if (r == i + 1) vr = mk<double>(1, 0);
-      else if (r >= i + 2) vr = mul(ld<double>(T.at(r, i)), scal);
-      st<double>(T.v + r, vr);
-    }
-    __syncthreads();
-    for (int r = i + 1 + tid; r < n; r += kThreads)
-      st<double>(T.at(r, i), r == i + 1 ? mk(beta, 0.0) : (keep ? ld<double>(T.v + r) : mk<double>(0, 0)));
-    if (tid == 0 && tau_out) tau_out[i] = double2{tau.re, tau.im};
-    // H <- H (I - tau v v^H): row r, columns i+1..n-1
-    for (int r = tid; r < n; r += kThreads) {
-      cx<double> w = mk<double>(0, 0);
-      for (int c = i + 1; c < n; ++c) w = add(w, mul(ld<double>(T.at(r, c)), ld<double>(T.v + c)));
-      const cx<double> tw = mul(tau, w);
-      for (int c = i + 1; c < n; ++c) st<double>(T.at(r, c), sub(ld<double>(T.at(r, c)), mulc(tw, ld<double>(T.v + c))));
-      if (Q) {
-        cx<double> wq = mk<double>(0, 0);
-        for (int c = i + 1; c < n; ++c) wq = add(wq, mul(Q->ld(r, c), ld<double>(T.v + c)));
-        const cx<double> twq = mul(tau, wq);
-        for (int c = i + 1; c < n; ++c) Q->st(r, c, sub(Q->ld(r, c), mulc(twq, ld<double>(T.v + c))));
-      }
-    }
-    __syncthreads();
-    // H <- (I - conj(tau) v v^H) H: column c, rows i+1..n-1
-    for (int c = i + 1 + tid; c < n; c += kThreads) {
-      cx<double> y = mk<double>(0, 0);
-      for (int k = i + 1; k < n; ++k) y = add(y, cmul(ld<double>(T.v + k), ld<double>(T.at(k, c))));
-      const cx<double> ty = cmul(tau, y);
-      for (int k = i + 1; k < n; ++k) st<double>(T.at(k, c), sub(ld<double>(T.at(k, c)), mul(ld<double>(T.v + k), ty)));
-    }
-    __syncthreads();
-  }
-}
-
-// Q <- Q H_0 H_1 ... H_{n-2} from the compact form in the tile (v(i+2:n)
-// below the subdiagonal, v(i+1) = 1) and tau (zunghr's product, formed
-// forward), Q in global memory.
-__device__ void unghr_tile(const Tile &T, Shared &sh, const GMat &Q, const double2 *tau) {
-  const int n = T.n, tid = threadIdx.x;
-  (void)sh;
-  for (int i = 0; i + 1 < n; ++i) {
-    const cx<double> ta = mk(tau[i].x, tau[i].y);
-    for (int r = tid; r < n; r += kThreads) {
-      auto v = [&](int c) { return c == i + 1 ? mk<double>(1, 0) : ld<double>(T.at(c, i)); };
-      cx<double> w = mk<double>(0, 0);
-      for (int c = i + 1; c < n; ++c) w = add(w, mul(Q.ld(r, c), v(c)));
-      const cx<double> tw = mul(ta, w);
-      for (int c = i + 1; c < n; ++c) Q.st(r, c, sub(Q.ld(r, c), mulc(tw, v(c))));
-    }
-  }
-  __syncthreads();
-}
-
-// ---------------------------------------------------------------------------
-// QR iteration on the tile (upper Hessenberg, real subdiagonal after
-// make_real) with the Schur vectors Z in global memory (thread r: row r,
-// n <= kThreads; each thread carries Z(r, K+1) in a register from one bulge
-// step to the next and loads the following column one step ahead).  Returns
-// the count of eigenvalues accepted at the iteration cap.
-// ---------------------------------------------------------------------------
-__device__ int lahqr_tile(const Tile &T, Shared &sh, const GMat &Z, int itmax, bool make_real) {
-  const int n = T.n, tid = threadIdx.x;
-  const double ulp = DBL_EPSILON;
-  const double smlnum = DBL_MIN * (double(n > 0 ? n : 1) / ulp);
-  auto H = [&](int r, int c) { return ld<double>(T.at(r, c)); };
-  if (make_real) {
-    for (int i = 1; i < n; ++i) {
-      const cx<double> h = H(i, i - 1);
-      if (h.im != 0.0) {  // uniform: every thread reads the same entry
-        const double d1 = cabs1(h);
-        const cx<double> w = scale(h, frcp(d1));
-        const cx<double> sc = scale(conj(w), frsq(abs2(w)));  // conj(h/|h|)
-        __syncthreads();
-        if (tid == 0) st<double>(T.at(i, i - 1), mk(fsqrt(abs2(h)), 0.0));
-        for (int x = i + tid; x < n; x += kThreads) st<double>(T.at(i, x), mul(H(i, x), sc));
-        for (int x = tid; x <= i + 1 && x < n; x += kThreads)
-          if (x != i) st<double>(T.at(x, i), mulc(H(x, i), sc));
-        __syncthreads();
-        if (tid == 0) st<double>(T.at(i, i), mulc(H(i, i), sc));
-        for (int r = tid; r < n; r += kThreads) Z.st(r, i, mulc(Z.ld(r, i), sc));
-        __syncthreads();
-      }
-    }
-  }
-  int I = n - 1, L = 0, its = 0, nfail = 0;
-  while (I >= 0) {
-    // ---- deflation: the largest negligible k in L+1..I, as the reference's
-    // scan from I down to L+1 finds it (each thread tests its k's) ----
-    int best = 0;
-    for (int k = L + 1 + tid; k <= I; k += kThreads) {
-      const cx<double> h = H(k, k - 1);
-      bool nk = cabs1(h) <= smlnum;
-      if (!nk) {
-        const cx<double> hkk1 = H(k - 1, k - 1), hkk = H(k, k);
-        double tst = cabs1(hkk1) + cabs1(hkk);
-        if (tst == 0.0) {
-          if (k - 2 >= 0) tst += fabs(H(k - 1, k - 2).re);
-          if (k + 1 <= n - 1) tst += fabs(H(k + 1, k).re);
-        }
-        if (fabs(h.re) <= ulp * tst) {
-          const cx<double> hup = H(k - 1, k);
-          const double ab = fmax(cabs1(h), cabs1(hup)), ba = fmin(cabs1(h), cabs1(hup));
-          const double d3 = cabs1(sub(hkk1, hkk));
-          const double aa = fmax(cabs1(hkk), d3), bb = fmin(cabs1(hkk), d3);
-          const double s = aa + ab;
-          nk = ba * (ab / s) <= fmax(smlnum, ulp * (bb * (aa / s)));
-        }
-      }
-      if (nk) best = k;
-    }
-    const int Lf = block_max_index(best > 0, best, sh);
-    if (its > itmax) {
-      ++nfail;  // accepted without convergence (the reference's silent case)
-      --I;
-      L = 0;
-      its = 0;
-      continue;
-    }
-    if (Lf > L) {
-      L = Lf;
-      if (tid == 0) st<double>(T.at(L, L - 1), mk<double>(0, 0));
-      __syncthreads();
-    }
-    if (L >= I) {
-      --I;
-      L = 0;
-      its = 0;
-      continue;
-    }
-    // ---- shift and first column (every thread computes the same) ----
-    cx<double> t;
-    if (its == 10) {
-      t = H(L, L);
-      t.re += 0.75 * fabs(H(L + 1, L).re);
-    } else if (its == 20) {
-      t = H(I, I);
-      t.re += 0.75 * fabs(H(I, I - 1).re);
-    } else {
-      t = H(I, I);
-      const cx<double> u2 = mul(H(I - 1, I), H(I, I - 1));
-      if (u2.re != 0.0 || u2.im != 0.0) {
-        const cx<double> x = scale(sub(H(I - 1, I - 1), t), 0.5);
-        const double sx = cabs1(x);
-        const double s = fmax(fsqrt(cabs1(u2)), sx);
-        const double is = frcp(s);
-        const cx<double> xs = scale(x, is);
-        cx<double> ys = csqrt(add(mul(xs, xs), scale(u2, is * is)));
-        if (sx > 0.0 && xs.re * ys.re + xs.im * ys.im < 0.0) ys = mk(-ys.re, -ys.im);
-        t = sub(t, mul(scale(u2, is), inv(add(xs, ys))));
-      }
-    }
-    const cx<double> h11s = sub(H(L, L), t);
-    const double h21 = H(L + 1, L).re;
-    const double is0 = frcp(cabs1(h11s) + fabs(h21));
-    const cx<double> a0 = scale(h11s, is0);
-    const double a1 = h21 * is0;
-    // ---- the sweep; each thread carries Z(r, K+1) of its row between steps ----
-    cx<double> zk1 = tid < n ? Z.ld(tid, L) : mk<double>(0, 0);
-    for (int K = L; K < I; ++K) {
-      cx<double> b0 = mk(a0.re, a0.im);
-      double b1 = a1;
-      if (K > L) {
-        b0 = H(K, K - 1);
-        b1 = H(K + 1, K - 1).re;
-      }
-      double nb0, nrm2;
-      Rot<double> q = rot2(b0, b1, nb0, nrm2);
-      if (nrm2 == 0.0) {  // G = I
-        q.c = mk<double>(1, 0);
-        q.s = 0.0;
-        nb0 = 0.0;
-      }
-      const cx<double> znext = tid < n ? Z.ld(tid, K + 1) : mk<double>(0, 0);
-      // rows K, K+1 over columns K..n-1
-      for (int c = K + tid; c < n; c += kThreads) {
-        cx<double> h1 = H(K, c), h2 = H(K + 1, c);
-        rot_left(q, h1, h2);
-        st<double>(T.at(K, c), h1);
-        st<double>(T.at(K + 1, c), h2);
-      }
-      __syncthreads();
-      if (K > L && tid == kThreads - 1) {
-        st<double>(T.at(K, K - 1), mk(nb0, 0.0));
-        st<double>(T.at(K + 1, K - 1), mk<double>(0, 0));
-      }
-      // columns K, K+1 over rows 0..min(K+2, I)
-      const int i3 = (K + 2) < I ? (K + 2) : I;
-      for (int r = tid; r <= i3; r += kThreads) {
-        cx<double> h1 = H(r, K), h2 = H(r, K + 1);
-        rot_right(q, h1, h2);
-        st<double>(T.at(r, K), h1);
-        st<double>(T.at(r, K + 1), h2);
-      }
-      // Schur vectors: columns K, K+1 of row tid
-      if (tid < n) {
-        cx<double> z0 = zk1, z1 = znext;
-        rot_right(q, z0, z1);
-        Z.st(tid, K, z0);
-        zk1 = z1;
-      }
-      __syncthreads();
-    }
-    if (tid < n) Z.st(tid, I, zk1);
-    // ---- make H(I, I-1) real (Toolbox.hpp:337-367) ----
-    const cx<double> h = H(I, I - 1);
-    __syncthreads();
-    if (h.im != 0.0 && abs2(h) > 0.0) {
-      const double id = frsq(abs2(h));
-      const double d = abs2(h) * id;
-      const cx<double> zz = mk(h.re * id, -h.im * id);  // conj(h/|h|)
-      if (tid == 0) st<double>(T.at(I, I - 1), mk(d, 0.0));
-      for (int x = I + 1 + tid; x < n; x += kThreads) st<double>(T.at(I, x), mul(H(I, x), zz));
-      for (int x = tid; x < I; x += kThreads) st<double>(T.at(x, I), mulc(H(x, I), zz));
-      for (int r = tid; r < n; r += kThreads) Z.st(r, I, mulc(Z.ld(r, I), zz));
-    }
-    ++its;
-    __syncthreads();
-  }
-  return nfail;
-}
-
-// ---------------------------------------------------------------------------
-// Eigenvectors of the triangular tile (ztrevc + backsubstitution): thread k
-// solves for eigenvector k with the reference's small-pivot clamp and leaves
-// y = -x in column k above the diagonal; then R <- R X in global memory,
-// thread r owning row r (column k of R X = R [x; 1; 0], the reference's
-// scaling).  Returns nothing; lam(k) = T(k, k) stays on the diagonal.
-// ---------------------------------------------------------------------------
-__device__ void trevc_tile(const Tile &T, const GMat &R) {
-  const int n = T.n, tid = threadIdx.x;
-  const double ulp = DBL_EPSILON;
-  const double smlnum = DBL_MIN * (double(n > 0 ? n : 1) / ulp);
-  for (int j = n - 2; j >= 0; --j) {
-    const cx<double> tjj = ld<double>(T.at(j, j));
-    for (int r = j + 1 + tid; r < n; r += kThreads) {
-      const cx<double> lam = ld<double>(T.at(r, r));
-      const double smin = fmax(ulp * cabs1(lam), smlnum);
-      cx<double> d = sub(tjj, lam);
-      if (cabs1(d) < smin) d = mk(smin, 0.0);
-      const cx<double> yj = mul(ld<double>(T.at(j, r)), inv(d));
-      st<double>(T.at(j, r), yj);
-      for (int i = 0; i < j; ++i) st<double>(T.at(i, r), sub(ld<double>(T.at(i, r)), mul(ld<double>(T.at(i, j)), yj)));
-    }
-    __syncthreads();
-  }
-  // R(r, k) <- R(r, k) - sum_{j<k} R(r, j) y(j, k), from the last column
-  for (int r = tid; r < n; r += kThreads)
-    for (int k = n - 1; k >= 1; --k) {
-      cx<double> acc = R.ld(r, k);
-      for (int j = 0; j < k; ++j) acc = sub(acc, mul(R.ld(r, j), ld<double>(T.at(j, k))));
-      R.st(r, k, acc);
-    }
-}
-
-// ---------------------------------------------------------------------------
-// kernels
-// ---------------------------------------------------------------------------
 struct BigArgs {
-  double *rA, *iA;  // A / H / T (in place for the stages)
+  double *rA, *iA;  // A / H / T
   double *rB, *iB;  // V / Q / Z / R
   double *rE, *iE;  // E / tau
   int32_t *info;
   Geom G;
   int itmax;
-  int mode;
   uint32_t flags;
+  const int32_t *list, *list_count;  // fused: only these matrices
+  const double *rC, *iC;             // roots: the coefficients
 };
 
-__device__ GMat gmat(double *re, double *im, const Geom &G, int64_t m) {
-  return GMat{re, im, G.mat_base(m), G.T, (int64_t)G.n * G.T};
+// the matrix of this workgroup, from the batch or the list (whose length is
+// only known on the device: the workgroups past it find none)
+__device__ __forceinline__ bool block_matrix(const BigArgs &a, int64_t &m) {
+  if (a.list) {
+    const int64_t cnt = *a.list_count, b = blockIdx.x;
+    m = b < cnt ? a.list[xcd_remap(b, cnt)] : 0;
+    return b < cnt;
+  }
+  m = xcd_block();
+  return m < a.G.nmat;
 }
 
-__global__ __launch_bounds__(kThreads) void k_big(BigArgs a) {
+// ---------------------------------------------------------------------------
+// reduction
+// ---------------------------------------------------------------------------
+enum { RD_FUSED = 0, RD_GEHRD = 1, RD_HESS = 2, RD_UNGHR = 3 };
+
+template <int CAP, int W, int MODE>
+__global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce(BigArgs a) {
+  using S = ReduceBlock<CAP, W>;
   extern __shared__ double2 lds[];
-  __shared__ Shared sh;
-  const int n = a.G.n, tid = threadIdx.x;
-  Tile T;
-  T.n = n;
-  T.ld = n + 1;
-  T.t = lds;
-  T.v = lds + n * (n + 1);
-  double2 *tau = T.v + n;  // n entries
-  for (int64_t m = blockIdx.x; m < a.G.nmat; m += gridDim.x) {
-    const GMat A = gmat(a.rA, a.iA, a.G, m);
-    const GMat B = gmat(a.rB, a.iB, a.G, m);
-    const int64_t vb = a.G.vec_base(m);
-    // the matrix into the tile (full; the QR and eigenvector stages read the
-    // Hessenberg part or the upper triangle only)
-    for (int c = 0; c < n; ++c)
-      for (int r = tid; r < n; r += kThreads) {
-        cx<double> x = A.ld(r, c);
-        if ((a.mode == BIG_LAHQR && r > c + 1) || (a.mode == BIG_TREVC && r > c)) x = mk<double>(0, 0);
-        st<double>(T.at(r, c), x);
-      }
-    if (a.mode == BIG_UNGHR)
-      for (int i = tid; i < n; i += kThreads)
-        tau[i] = i + 1 < n ? double2{a.rE[vb + a.G.ve(i)], a.iE[vb + a.G.ve(i)]} : double2{0, 0};
-    // Q or Z starts as the identity where this kernel forms it
-    if (a.mode == BIG_FUSED || a.mode == BIG_HESS || a.mode == BIG_UNGHR) {
-      const GMat &Q = a.mode == BIG_UNGHR ? A : B;
-      for (int c = 0; c < n; ++c)
-        for (int r = tid; r < n; r += kThreads) Q.st(r, c, mk<double>(r == c ? 1.0 : 0.0, 0));
-    }
+  S &sm = *reinterpret_cast<S *>(lds);
+  double2 *tau = lds + sizeof(S) / sizeof(double2);
+  int64_t m;
+  if (!block_matrix(a, m)) return;  // workgroup-uniform
+  const int n = a.G.n, tid = threadIdx.x, r = tid % CAP, q = tid / CAP;
+  const int64_t base = a.G.mat_base(m), vb = a.G.vec_base(m);
+  reduce_load(sm, n, a.G, base, a.rA, a.iA);
+  if constexpr (MODE == RD_UNGHR) {
+    if (tid + 1 < n) st<double>(tau + tid, mk<double>(a.rE[vb + a.G.ve(tid)], a.iE[vb + a.G.ve(tid)]));
     __syncthreads();
-    if (a.mode == BIG_GEHRD || a.mode == BIG_HESS) {
-      reduce_tile(T, sh, true, a.mode == BIG_HESS ? &B : nullptr, tau);
-      for (int c = 0; c < n; ++c)
-        for (int r = tid; r < n; r += kThreads) A.st(r, c, ld<double>(T.at(r, c)));
-      if (a.rE)
-        for (int i = tid; i + 1 < n; i += kThreads) {
-          a.rE[vb + a.G.ve(i)] = tau[i].x;
-          a.iE[vb + a.G.ve(i)] = tau[i].y;
-        }
-    } else if (a.mode == BIG_UNGHR) {
-      unghr_tile(T, sh, A, tau);
-    } else if (a.mode == BIG_LAHQR) {
-      const int nfail = lahqr_tile(T, sh, B, a.itmax, true);
-      for (int c = 0; c < n; ++c)
-        for (int r = tid; r < n; r += kThreads) A.st(r, c, r <= c ? ld<double>(T.at(r, c)) : mk<double>(0, 0));
-      for (int r = tid; r < n; r += kThreads) {
-        const double2 d = *T.at(r, r);
-        a.rE[vb + a.G.ve(r)] = d.x;
-        a.iE[vb + a.G.ve(r)] = d.y;
-      }
-      if (a.info && tid == 0) a.info[m] = nfail;
-    } else if (a.mode == BIG_TREVC) {
-      trevc_tile(T, B);
-    } else {  // BIG_FUSED: A read only (unless the Schur form is asked for)
-      reduce_tile(T, sh, false, &B, nullptr);
-      const int nfail = lahqr_tile(T, sh, B, a.itmax, false);
-      if (a.flags & VEIG_WRITE_SCHUR)
-        for (int c = 0; c < n; ++c)
-          for (int r = tid; r < n; r += kThreads) A.st(r, c, r <= c ? ld<double>(T.at(r, c)) : mk<double>(0, 0));
-      for (int r = tid; r < n; r += kThreads) {
-        const double2 d = *T.at(r, r);
-        a.rE[vb + a.G.ve(r)] = d.x;
-        a.iE[vb + a.G.ve(r)] = d.y;
-      }
-      __syncthreads();
-      trevc_tile(T, B);
-      if (a.info && tid == 0) a.info[m] = nfail;
+  } else {
+    reduce_block(sm, n, tau);
+    const bool fused = MODE == RD_FUSED;
+    reduce_store(sm, n, a.G, base, fused ? a.rB : a.rA, fused ? a.iB : a.iA);
+    if (a.rE && tid + 1 < n) {
+      const cx<double> t = ld<double>(tau + tid);
+      a.rE[vb + a.G.ve(tid)] = t.re;
+      a.iE[vb + a.G.ve(tid)] = t.im;
     }
-    __syncthreads();  // the tile is reused by the next matrix
+  }
+  if constexpr (MODE == RD_HESS || MODE == RD_UNGHR) {
+    cx<double> z[S::CH];
+    form_q_block(sm, n, tau, z);
+    double *re = MODE == RD_HESS ? a.rB : a.rA, *im = MODE == RD_HESS ? a.iB : a.iA;
+#pragma unroll
+    for (int j = 0; j < S::CH; ++j) {
+      const int c = q * S::CH + j;
+      if (q < W && r < n && c < n) {
+        const int64_t idx = base + a.G.el(r, c);
+        re[idx] = z[j].re;
+        im[idx] = z[j].im;
+      }
+    }
   }
 }
 
-size_t big_lds_bytes(int n) { return (size_t)(n * (n + 1) + 2 * n) * sizeof(double2); }
+// ---------------------------------------------------------------------------
+// QR iteration, Schur vectors, eigenvectors
+// ---------------------------------------------------------------------------
+enum { SC_FUSED = 0, SC_LAHQR = 1, SC_TREVC = 2, SC_ROOTS = 3 };
+
+template <int SL, int NT>
+constexpr int schur_threads() {
+  constexpr int RW = SchurRows<SL, NT>::RW;
+  return 64 * (1 + (SL * NT + RW - 1) / RW);
+}
+
+// wavefronts per SIMD the register allocation is held to
+template <int SL>
+constexpr int schur_waves() { return SL <= 24 ? 4 : 3; }
+
+template <int SL, int NT, int MODE>
+__global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_waves_per_eu(schur_waves<SL>()))) void k_schur(BigArgs a) {
+  using Rows = SchurRows<SL, NT>;
+  using Ring = typename Rows::Ring;
+  constexpr int CAP = Rows::CAP, P = (CAP + 63) / 64;
+  extern __shared__ double2 lds[];
+  Ring &ring = *reinterpret_cast<Ring *>(lds);
+  const BandTile t{MODE == SC_TREVC ? lds : lds + sizeof(Ring) / sizeof(double2)};
+  int64_t m;
+  if (!block_matrix(a, m)) return;  // workgroup-uniform
+  const int n = a.G.n, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), zw = (blockDim.x >> 6) - 1;
+  const int64_t base = a.G.mat_base(m), vb = a.G.vec_base(m);
+  // the band (Hessenberg part, or upper triangle) from memory, by every wavefront
+  for (int i = threadIdx.x; i < BandTile::entries(n); i += blockDim.x) st<double>(t.h + i, mk<double>(0, 0));
+  __syncthreads();
+  if constexpr (MODE == SC_ROOTS) {
+    // the companion matrix of c_0 + ... + c_n x^n (create_companion_matrices,
+    // Toolbox.hpp:605-643): ones below the diagonal, -c_r / c_n in the last
+    // column (Smith's division)
+    const int64_t cb = a.G.vec_base(m, 1) + (m / a.G.T) * a.G.T;  // slots of n + 1 entries
+    const cx<double> lead = mk<double>(a.rC[cb + n * a.G.T], a.iC[cb + n * a.G.T]);
+    for (int r = threadIdx.x; r < n; r += blockDim.x) {
+      const cx<double> c = cdiv(mk<double>(a.rC[cb + r * a.G.T], a.iC[cb + r * a.G.T]), lead);
+      if (r >= 1) st<double>(t.at(r, r - 1), mk<double>(1, 0));
+      st<double>(t.at(r, n - 1), mk(-c.re, -c.im));
+    }
+  } else {
+    const double *re = MODE == SC_FUSED ? a.rB : a.rA, *im = MODE == SC_FUSED ? a.iB : a.iA;
+    constexpr int sub = MODE == SC_TREVC ? 0 : 1;
+    for (int c = threadIdx.x >> 6; c < n; c += zw + 1)
+      for (int r = lane; r <= c + sub && r < n; r += 64) {
+        const int64_t idx = base + a.G.el(r, c);
+        st<double>(t.at(r, c), mk<double>(re[idx], im[idx]));
+      }
+  }
+  int hw = 0;  // the wavefront of the iteration; zi: this one among the others
+  if constexpr (MODE == SC_TREVC) __syncthreads();
+  else hw = chain_wave(ring.simd);
+  const int zi = w < hw ? w : w - 1;
+  if (w == hw) {
+    // ---------------- the iteration and the eigenvector solve ----------------
+    __builtin_amdgcn_s_setprio(3);  // the workgroup waits for the chain: it issues first on its SIMD
+    if constexpr (MODE != SC_TREVC) {
+      if constexpr (MODE == SC_LAHQR) {
+        make_subdiag_real(t, n, lane, &ring.step[1][0].c);
+        __syncthreads();  // its phases are out
+      }
+      const int nfail = lahqr_stream<P, true>(t, n, lane, ring, a.itmax);
+      for (int r = lane; r < n; r += 64) {
+        const cx<double> e = ld<double>(t.at(r, r));
+        a.rE[vb + a.G.ve(r)] = e.re;
+        a.iE[vb + a.G.ve(r)] = e.im;
+      }
+      if (a.info && lane == 0) a.info[m] = nfail;
+      if (MODE != SC_FUSED || (a.flags & VEIG_WRITE_SCHUR))
+        for (int c = 0; c < n; ++c)
+          for (int r = lane; r < n; r += 64) {
+            const int64_t idx = base + a.G.el(r, c);
+            const cx<double> x = r <= c ? ld<double>(t.at(r, c)) : mk<double>(0, 0);
+            a.rA[idx] = x.re;
+            a.iA[idx] = x.im;
+          }
+    }
+    if constexpr (MODE == SC_FUSED || MODE == SC_TREVC) {
+      trevc_rows<P>(t, n, lane);
+      __syncthreads();  // the eigenvector factor is ready
+    }
+  } else {
+    // ---------------- the Schur vectors ----------------
+    Rows z;
+    z.init(lane);
+    const int row0 = zi * Rows::RW, row = row0 + z.rl;
+    if constexpr (MODE == SC_FUSED) {
+      // the stages: the slots beside the one that the iteration is writing,
+      // each as two vectors
+      static_assert(schur_threads<SL, NT>() / 64 - 1 <= 2 * NT, "a stage for each wavefront");
+      double2 *stage = &ring.step[1][0].c + zi * CAP;
+      z.form_q(row, n, a.G, base, vb, a.rB, a.iB, a.rE, a.iE, stage);
+    } else if constexpr (MODE == SC_ROOTS) {
+#pragma unroll
+      for (int c = 0; c < SL; ++c) z.z[c] = mk<double>(SL * z.h + c == row ? 1.0 : 0.0, 0);
+    } else {
+      z.load(row, n, a.G, base, a.rB, a.iB);
+    }
+    if constexpr (MODE == SC_LAHQR) {
+      __syncthreads();  // the phases that made the subdiagonal real
+#pragma unroll
+      for (int c = 0; c < SL; ++c)
+        if (SL * z.h + c < n) z.z[c] = mulc(z.z[c], ld<double>(&ring.step[1][0].c + SL * z.h + c));
+    }
+    if constexpr (MODE != SC_TREVC) {
+      z.start(ring, zi, zw);
+      z.replay(ring);
+    }
+    if constexpr (MODE == SC_FUSED || MODE == SC_TREVC) {
+      __syncthreads();  // the eigenvector factor is ready
+      backtransform_mfma(t, z, row0, n, a.G, base, a.rB, a.iB);
+    } else {
+      z.store(row, n, a.G, base, a.rB, a.iB);
+    }
+  }
+}
+
+int set_lds(const void *kernel, size_t bytes) {
+  if (bytes > 64 * 1024)
+    VEIG_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+  return VEIG_OK;
+}
+
+template <int CAP, int W, int MODE>
+int launch_reduce(const BigArgs &a, hipStream_t s) {
+  using S = ReduceBlock<CAP, W>;
+  const size_t bytes = sizeof(S) + CAP * sizeof(double2);  // and tau
+  VEIG_TRY(set_lds((const void *)k_reduce<CAP, W, MODE>, bytes));
+  hipLaunchKernelGGL((k_reduce<CAP, W, MODE>), dim3((unsigned)a.G.nmat), dim3(S::kThreads), bytes, s, a);
+  VEIG_HIP(hipGetLastError());
+  return VEIG_OK;
+}
+
+template <int MODE>
+int reduce_for(const BigArgs &a, hipStream_t s) {
+  if (a.G.n <= 48) return launch_reduce<48, 4, MODE>(a, s);
+  if (a.G.n <= 64) return launch_reduce<64, 4, MODE>(a, s);
+  if (a.G.n <= 80) return launch_reduce<80, 8, MODE>(a, s);
+  return launch_reduce<96, 6, MODE>(a, s);
+}
+
+template <int SL, int NT, int MODE>
+int launch_schur(const BigArgs &a, hipStream_t s) {
+  using Rows = SchurRows<SL, NT>;
+  const size_t bytes =
+      (MODE == SC_TREVC ? 0 : sizeof(typename Rows::Ring)) + (size_t)BandTile::entries(a.G.n) * sizeof(double2);
+  const unsigned threads = 64u * (1 + (a.G.n + Rows::RW - 1) / Rows::RW);
+  VEIG_TRY(set_lds((const void *)k_schur<SL, NT, MODE>, bytes));
+  hipLaunchKernelGGL((k_schur<SL, NT, MODE>), dim3((unsigned)a.G.nmat), dim3(threads), bytes, s, a);
+  VEIG_HIP(hipGetLastError());
+  return VEIG_OK;
+}
+
+template <int MODE>
+int schur_for(const BigArgs &a, hipStream_t s) {
+  if (a.G.n <= 40) return launch_schur<20, 2, MODE>(a, s);
+  if (a.G.n <= 48) return launch_schur<24, 2, MODE>(a, s);
+  if (a.G.n <= 64) return launch_schur<32, 2, MODE>(a, s);
+  if (a.G.n <= 80) return launch_schur<20, 4, MODE>(a, s);
+  return launch_schur<24, 4, MODE>(a, s);
+}
 
 }  // namespace
 
 namespace veig {
 
-// The kernel above for one batch (mode: what it computes, see BigArgs).
 int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, double *iB, double *rE, double *iE,
-               int32_t *info, int itmax, uint32_t flags, hipStream_t s) {
+               int32_t *info, int itmax, uint32_t flags, hipStream_t s, const int32_t *list,
+               const int32_t *list_count, const double *rC, const double *iC) {
   if (G.n > VEIG_MAX_DIM) return fail(VEIG_ERR_UNSUPPORTED, "order beyond VEIG_MAX_DIM");
-  const size_t bytes = big_lds_bytes(G.n);
-  VEIG_HIP(hipFuncSetAttribute((const void *)k_big, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-  int dev = 0, cus = 256;
-  VEIG_HIP(hipGetDevice(&dev));
-  VEIG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  const int per_cu = (int)(160 * 1024 / (bytes + 1024)) > 0 ? (int)(160 * 1024 / (bytes + 1024)) : 1;
-  const int64_t want = (int64_t)cus * per_cu;
-  const unsigned grid = (unsigned)(G.nmat < want ? G.nmat : want);
-  BigArgs a{rA, iA, rB, iB, rE, iE, info, G, itmax > 0 ? itmax : 30, mode, flags};
-  hipLaunchKernelGGL(k_big, dim3(grid), dim3(kThreads), bytes, s, a);
-  VEIG_HIP(hipGetLastError());
-  return VEIG_OK;
+  if (G.nmat > INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
+  const BigArgs a{rA, iA, rB, iB, rE, iE, info, G, itmax > 0 ? itmax : 30, flags, list, list_count, rC, iC};
+  switch (mode) {
+    case BIG_FUSED:
+      VEIG_TRY(reduce_for<RD_FUSED>(a, s));
+      return schur_for<SC_FUSED>(a, s);
+    case BIG_GEHRD: return reduce_for<RD_GEHRD>(a, s);
+    case BIG_HESS: return reduce_for<RD_HESS>(a, s);
+    case BIG_UNGHR: return reduce_for<RD_UNGHR>(a, s);
+    case BIG_LAHQR: return schur_for<SC_LAHQR>(a, s);
+    case BIG_TREVC: return schur_for<SC_TREVC>(a, s);
+    default:  // BIG_ROOTS: orders up to VEIG_MAX_DIM_FAST
+      return G.n <= 48 ? launch_schur<24, 2, SC_ROOTS>(a, s) : launch_schur<32, 2, SC_ROOTS>(a, s);
+  }
 }
 
 }  // namespace veig

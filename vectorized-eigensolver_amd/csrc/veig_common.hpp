@@ -287,24 +287,6 @@ __device__ __forceinline__ void zgeev_wave(const FusedArgs &a, Tiles<R, NB, P> &
   gehrd_q<R, NB, P>(g, z, nmax, true, false, nullptr);
   const int nfail = lahqr<R, NB, P>(g, z, a.itmax, false);
   if (a.flags & VEIG_WRITE_SCHUR) store_rows<R, NB, P>(g, a.G, base, a.rA, a.iA);
-  if constexpr (NB == 64) {
-    // one matrix per wavefront: eigenvector solves in LDS, V streamed out
-    static_assert(OUT == OUT_V && P == 1, "one matrix per wavefront: FP64, one index per lane");
-    const cx<R> lam = trevc_solve_lds<R, NB>(g, nmax);
-    backtransform_lds<R, NB>(g, z, nmax, [&](int k, cx<R> v) {
-      if (g.r < g.n) {
-        const int64_t idx = base + a.G.el(g.r, k);
-        a.rV[idx] = (double)v.re;
-        a.iV[idx] = (double)v.im;
-      }
-    });
-    if (g.r < g.n) {
-      a.rE[vbase + a.G.ve(g.r)] = (double)lam.re;
-      a.iE[vbase + a.G.ve(g.r)] = (double)lam.im;
-    }
-    if (a.info && valid && g.r == 0) a.info[m] = nfail;
-    return;
-  }
   cx<R> lam[P];
   solve_eigvecs<R, NB, P>(g, nmax, lam);
   if constexpr (OUT == OUT_ZXY) {
@@ -405,20 +387,22 @@ inline void launch_one(const FusedArgs &a, hipStream_t s) {
   hipLaunchKernelGGL((k_zgeev<R, NB, P, OUT>), dim3((unsigned)grid), dim3(64), 0, s, a);
 }
 
-// orders 33..64, one matrix per two-wavefront workgroup (instantiated for
-// <double, OUT_V>, <float, OUT_V> and <float, OUT_VW>)
-template <typename R, int OUT>
+// complex64 at orders 33..64, one matrix per two-wavefront workgroup
+// (instantiated for OUT_V and OUT_VW)
+template <int OUT>
 int launch_zgeev64(const FusedArgs &a, hipStream_t s);
 
-// Orders beyond the lane-group kernels (veig_big.hip): one workgroup per
-// matrix, the matrix in LDS, the unitary factor in global memory.  Modes:
-// the fused eigendecomposition (A read only; Q, Z and then V in B; E), and
-// the stage entries in place: zgehrd (A -> compact form, tau in E),
-// hessenberg (also Q in B), zunghr (reflectors in A, tau in E -> Q in A),
-// zlahqr (H in A -> T, Z in B updated, E), ztrevc (T in A, B <- B X).
-enum { BIG_FUSED = 0, BIG_GEHRD = 1, BIG_HESS = 2, BIG_UNGHR = 3, BIG_LAHQR = 4, BIG_TREVC = 5 };
+// FP64 beyond the lane-group kernels (veig_big.hip), one matrix per
+// workgroup.  Modes: the fused eigendecomposition (A read only; Q, Z and then
+// V in B; E), of the batch or of a list of its matrices; the stage entries in
+// place: zgehrd (A -> compact form, tau in E), hessenberg (also Q in B),
+// zunghr (reflectors in A, tau in E -> Q in A), zlahqr (H in A -> T, Z in B
+// updated, E), ztrevc (T in A, B <- B X); polynomial roots with their Schur
+// form (coefficients in C -> T in A, Z in B, E).
+enum { BIG_FUSED = 0, BIG_GEHRD = 1, BIG_HESS = 2, BIG_UNGHR = 3, BIG_LAHQR = 4, BIG_TREVC = 5, BIG_ROOTS = 6 };
 int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, double *iB, double *rE, double *iE,
-               int32_t *info, int itmax, uint32_t flags, hipStream_t s);
+               int32_t *info, int itmax, uint32_t flags, hipStream_t s, const int32_t *list = nullptr,
+               const int32_t *list_count = nullptr, const double *rC = nullptr, const double *iC = nullptr);
 
 // FP64 batches and lists of orders up to NB on lane groups of LW lanes
 // (0: NB): Hessenberg reduction, then the QR iteration and eigenvectors on
@@ -433,13 +417,12 @@ template <typename R, int OUT = OUT_V>
 int launch_zgeev(const FusedArgs &a, hipStream_t s) {
   constexpr bool f32 = std::is_same<R, float>::value;
   if (a.G.nmat > (int64_t)INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
-  if (a.G.n > 64) {
-    if constexpr (!f32 && OUT == OUT_V) {
-      if (!a.mask && !a.list)
-        return launch_big(BIG_FUSED, a.G, a.rA, a.iA, a.rV, a.iV, a.rE, a.iE, a.info, a.itmax, a.flags, s);
-    }
-    return fail(VEIG_ERR_UNSUPPORTED, "orders above 64: FP64 whole batches only");
+  if constexpr (!f32 && OUT == OUT_V) {
+    if (a.G.n > 32 && !a.mask)
+      return launch_big(BIG_FUSED, a.G, a.rA, a.iA, a.rV, a.iV, a.rE, a.iE, a.info, a.itmax, a.flags, s, a.list,
+                        a.list_count);
   }
+  if (a.G.n > 64) return fail(VEIG_ERR_UNSUPPORTED, "orders above 64: FP64 only");
   const int nb = nb_for(a.G.n);
   switch (nb) {
     case 8:
@@ -461,8 +444,8 @@ int launch_zgeev(const FusedArgs &a, hipStream_t s) {
       launch_one<R, 32, 1, OUT>(a, s);
       break;
     default:
-      if constexpr (OUT == OUT_V || (f32 && OUT == OUT_VW)) {
-        return launch_zgeev64<R, OUT>(a, s);
+      if constexpr (f32 && (OUT == OUT_V || OUT == OUT_VW)) {
+        return launch_zgeev64<OUT>(a, s);
       } else {
         return fail(VEIG_ERR_UNSUPPORTED, "this output form handles orders up to 32");
       }

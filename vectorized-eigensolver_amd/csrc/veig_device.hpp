@@ -231,20 +231,6 @@ __device__ __forceinline__ R group_sum(R x) {
   return x;
 }
 
-// Call f(std::integral_constant<int, k>) for a wavefront-uniform runtime k in
-// [LO, HI): a binary tree of scalar branches, so that f can index register
-// arrays with a compile-time constant.
-template <int LO, int HI, typename F>
-__device__ __forceinline__ void uniform_dispatch(int k, F&& f) {
-  if constexpr (HI - LO <= 1) {
-    f(std::integral_constant<int, LO>{});
-  } else {
-    constexpr int MID = (LO + HI) / 2;
-    if (k < MID) uniform_dispatch<LO, MID>(k, f);
-    else uniform_dispatch<MID, HI>(k, f);
-  }
-}
-
 // f(integral_constant<int, I>) for I = 0 .. N-1 in order, unrolled
 template <typename F, int... Is>
 __device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, Is...>) {
@@ -657,9 +643,8 @@ VEIG_ZPIN_MULC(15, 164, 165, 166, 167)
 
 // Apply one bulge-chase rotation at row K to this lane's slots: rows K, K+1
 // of H over the lane's columns >= K, columns K, K+1 of H over the lane's rows
-// <= i3, and columns K, K+1 of the Schur vectors.  KC >= 0 is K as a
-// compile-time constant (unrolled sweeps); KC < 0 takes the wavefront-uniform
-// runtime Krt and selects the register columns by a uniform branch tree.
+// <= i3, and columns K, K+1 of the Schur vectors (KC: K as a compile-time
+// constant, the sweeps being unrolled).
 // The rotation's input is column K-1, rows K and K+1; at the first step of
 // a matrix's sweep (K = L) the caller has staged the shifted first column
 // (a0; a1 real) there -- in vsh[0..1] when L = 0 -- so that every step reads
@@ -669,11 +654,11 @@ VEIG_ZPIN_MULC(15, 164, 165, 166, 167)
 // rows >= L) and there are no Schur vectors.
 template <int KC, bool TZ = true, typename R, int NB, int P, int LAY, int LW>
 __device__ __forceinline__ void sweep_step(const Group<R, NB, P, LAY, LW>& g, cx<R> (&z)[P][NB], bool act,
-                                           int L, int I, int Krt = 0) {
+                                           int L, int I) {
   using L2 = typename Group<R, NB, P, LAY, LW>::L2;
   constexpr int LG = Group<R, NB, P, LAY, LW>::LG;
   const int n = g.n;
-  const int K = KC >= 0 ? KC : Krt;
+  constexpr int K = KC;
   constexpr int MPW = Group<R, NB, P, LAY, LW>::MPW;
   // with several matrices per wavefront, groups outside their sweep at this
   // K read the input (1, 0; 0) that lahqr keeps in vsh[2..3], whose rotation
@@ -681,8 +666,7 @@ __device__ __forceinline__ void sweep_step(const Group<R, NB, P, LAY, LW>& g, cx
   constexpr bool kIdle = TZ && MPW > 1;
   const L2* pb;
   if constexpr (KC == 0) pb = g.vsh;
-  else if constexpr (KC > 0) pb = g.at(KC, KC - 1);
-  else pb = K > 0 ? g.at(K, K - 1) : g.vsh;
+  else pb = g.at(KC, KC - 1);
   if constexpr (kIdle) pb = act ? pb : g.vsh + 2;
   // the row update's operands, loaded ahead of the rotation they wait for
   // (lanes outside the update read an entry of the tile and use none)
@@ -764,12 +748,7 @@ __device__ __forceinline__ void sweep_step(const Group<R, NB, P, LAY, LW>& g, cx
         for (int p = 0; p < P; ++p) rot_right(q, z[p][KK], z[p][KK + 1]);
       }
     };
-    if constexpr (!TZ) {
-    } else if constexpr (KC >= 0) {
-      zupd(std::integral_constant<int, KC>{});
-    } else {
-      uniform_dispatch<0, NB - 1>(K, zupd);
-    }
+    if constexpr (TZ) zupd(std::integral_constant<int, KC>{});
   }
   wave_sync();
 }
@@ -811,6 +790,7 @@ __device__ __forceinline__ int lahqr(const Group<R, NB, P, LAY, LW>& g, cx<R> (&
                                      bool make_real_subdiag) {
   constexpr int LG = Group<R, NB, P, LAY, LW>::LG;
   constexpr int MPW = Group<R, NB, P, LAY, LW>::MPW;
+  static_assert(MPW > 1, "several matrices share the wavefront");
   const int n = g.n;
   const R ulp = limits<R>::eps;
   const R smlnum = limits<R>::tiny * (R(n > 0 ? n : 1) / ulp);
@@ -1012,18 +992,11 @@ __device__ __forceinline__ int lahqr(const Group<R, NB, P, LAY, LW>& g, cx<R> (&
     wave_sync();
 
     // ---- the sweep (Toolbox.hpp:138-335), K = bulge row ----
-    if constexpr (MPW == 1) {
-      // one matrix per wavefront: a runtime loop over K, with the Schur
-      // vector columns selected by a uniform branch tree
-      static_assert(P == 1, "one matrix per wavefront uses one index per lane");
-      for (int K = kmin; K < kmax; ++K) sweep_step<-1, TZ>(g, z, ready && K >= L && K < I, L, I, K);
-    } else {
-      // steps kmin..kmax-1 of the wavefront, L..I-1 of this group
-      static_assert(NB <= 32, "step masks are 32 bits");
-      const unsigned kmask = kmax > kmin ? ((1u << kmax) - 1u) & ~((1u << kmin) - 1u) : 0u;
-      const unsigned amask = ready ? ((1u << I) - 1u) & ~((1u << L) - 1u) : 0u;
-      sweep_range<0, NB - 1, TZ>(g, z, amask, L, I, kmask);
-    }
+    // steps kmin..kmax-1 of the wavefront, L..I-1 of this group
+    static_assert(NB <= 32, "step masks are 32 bits");
+    const unsigned kmask = kmax > kmin ? ((1u << kmax) - 1u) & ~((1u << kmin) - 1u) : 0u;
+    const unsigned amask = ready ? ((1u << I) - 1u) & ~((1u << L) - 1u) : 0u;
+    sweep_range<0, NB - 1, TZ>(g, z, amask, L, I, kmask);
     if (ready && L > 0 && g.r == 0) {  // the staged first column
       st<R>(g.at(L, L - 1), mk<R>(0, 0));
       st<R>(g.at(L + 1, L - 1), mk<R>(0, 0));
@@ -1043,13 +1016,7 @@ __device__ __forceinline__ int lahqr(const Group<R, NB, P, LAY, LW>& g, cx<R> (&
           if (TZ && x > I && x < n) st<R>(g.at(I, x), mul(ld<R>(g.at(I, x)), zz));
           if (x < I && (TZ || x >= L)) st<R>(g.at(x, I), mulc(ld<R>(g.at(x, I)), zz));
         }
-        if constexpr (!TZ) {
-        } else if constexpr (MPW == 1) {
-          uniform_dispatch<0, NB>(I, [&](auto kc) {
-            constexpr int KK = decltype(kc)::value;
-            z[0][KK] = mulc(z[0][KK], zz);
-          });
-        } else {
+        if constexpr (TZ) {
 #pragma unroll
           for (int c = 1; c < NB; ++c)
             if (c == I) {
@@ -1216,8 +1183,7 @@ __device__ __forceinline__ void backtransform(const Group<R, NB, P>& g, cx<R> (&
 }
 
 // --------------------------------------------------------------------------
-// The same eigenvector solve for one matrix per wavefront (n up to 64, one
-// index per lane), with the right-hand sides kept in LDS instead of
+// The same eigenvector solve (one index per lane), with the right-hand sides kept in LDS instead of
 // registers: lane k keeps y = -x of its eigenvector in column k of the tile
 // (rows < k).  At step j lanes k > j read column j of T, which lane j only
 // starts to overwrite at step j-1, so T and the solutions share the tile.
@@ -1246,27 +1212,6 @@ __device__ __forceinline__ cx<R> trevc_solve_lds(const Group<R, NB, 1, LAY, LW>&
     wave_sync();
   }
   return lam;
-}
-
-// Row r of V = Z X from the tile left by trevc_solve_lds, one column at a
-// time, stored straight to the output (column k of V = Z [x; 1; 0]).
-template <typename R, int NB, typename Store>
-__device__ __forceinline__ void backtransform_lds(const Group<R, NB, 1>& g, const cx<R> (&z)[1][NB],
-                                                  int nmax, Store&& store) {
-  const int r = g.r;
-  // tile column r becomes -X(:, r): y above the diagonal, -1 on it, 0 below
-  if (r < g.n) {
-    st<R>(g.at(r, r), mk<R>(-1, 0));
-    for (int i = r + 1; i < g.n; ++i) st<R>(g.at(i, r), mk<R>(0, 0));
-  }
-  wave_sync();
-  for (int k = 0; k < nmax; ++k) {
-    cx<R> acc = mk<R>(0, 0);
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-      if (j < nmax) acc = add(acc, mul(z[0][j], ld<R>(g.at(j, k))));
-    store(k, mk(-acc.re, -acc.im));
-  }
 }
 
 template <typename R, int NB, int P>

@@ -1,8 +1,8 @@
-// Orders 33..64: one matrix per workgroup of two wavefronts.
+// complex64 at orders 33..64 (the first step of the mixed path, and
+// veig_zgeev_fp32): one matrix per workgroup of two wavefronts.
 //
 // At n = 64 a lane owning a row of the unitary factor needs 64 complex
-// doubles (256 registers) next to everything else, which does not fit.  So
-// the work is split by data:
+// values next to everything else.  So the work is split by data:
 //   * wavefront 0 (the Hessenberg engine) owns the Hessenberg / Schur matrix
 //     in LDS: it generates every reflector, applies it to H and runs the QR
 //     iteration (the same arithmetic and order as the lane-group kernels);
@@ -19,7 +19,7 @@
 #include <cstdint>
 #include <string>
 
-#include "veig_band.hpp"
+#include "veig_common.hpp"
 
 using namespace veig;
 
@@ -428,284 +428,25 @@ __device__ __forceinline__ void solve_one(const FusedArgs &a, LargeShared<R> &sh
 }
 
 // the batch, one matrix per workgroup
-template <typename R, int OUT>
+template <int OUT>
 __global__ __launch_bounds__(128) void k_zgeev64(FusedArgs a) {
-  __shared__ LargeShared<R> sh;
+  __shared__ LargeShared<float> sh;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t m = xcd_block();
   if (m >= a.G.nmat) return;  // workgroup-uniform
-  solve_one<R, OUT>(a, sh, m, w, lane);
-}
-
-// the matrices of a.list, on a persistent grid
-template <typename R, int OUT>
-__global__ __launch_bounds__(128) void k_zgeev64_list(FusedArgs a) {
-  __shared__ LargeShared<R> sh;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t cnt = *a.list_count;
-  for (int64_t i = blockIdx.x; i < cnt; i += gridDim.x) {
-    // an opaque copy of the lane: addresses derived from it are recomputed
-    // for every matrix instead of being hoisted out of the loop
-    int ln = lane;
-    asm volatile("" : "+v"(ln));
-    solve_one<R, OUT>(a, sh, a.list[i], w, ln);
-    __syncthreads();  // the tile and logs are reused by the next matrix
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Orders 33..64 in FP64, whole batches: two kernels.
-//
-// k_gehrd64 (four wavefronts per matrix on its dense tile, each owning 16
-// columns / rows of every update): the Hessenberg reduction alone, in
-// zgehrd's compact form -- H on and above the subdiagonal, the reflector
-// vectors v(i+2:n) below it, tau(i) -- written to the V and E planes, which
-// serve as its workspace.
-//
-// k_qr64 (one workgroup of three wavefronts per matrix): the QR iteration and
-// the eigenvectors with only the band row <= col + 2 of H in LDS (35 KB
-// instead of 66 KB) and the Schur-vector rows split over two wavefronts, two
-// lanes per row (each lane holds half a row, 32 complex values): wavefront 0
-// is the Hessenberg engine of k_zgeev64 on the banded tile; wavefronts 1 and
-// 2 (rows 0..31, 32..63) first form Q from the reflectors (Q <- Q H_i, the
-// row's two halves combined by a lane swap), then replay each recorded sweep;
-// the reflector on columns (31, 32) pairs the two halves of a row through the
-// same swap.  About 40 KB of LDS and ~170 registers per wavefront let four
-// matrices share a CU, against two for k_zgeev64.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(64 * reduce_waves<kN>()) void k_gehrd64(FusedArgs a) {
-  __shared__ ReduceTiles<kN> sm;
-  const int64_t m = xcd_block();
-  if (m >= a.G.nmat) return;  // workgroup-uniform
-  band_reduce_one<kN>(sm, a.G.n, a.G, a.G.mat_base(m), a.G.vec_base(m), a.G.n, a.rA, a.iA, a.rV, a.iV,
-                      a.rE, a.iE);
-}
-
-using GBand = Group<double, kN, 1, LAY_BAND>;
-
-struct QrShared64 {
-  double2 H[GBand::kSize + 1];
-  SweepLog<double> log[2];
-};
-
-// the other half of this lane's row (lane ^ 32)
-__device__ __forceinline__ cx<double> half_swap(cx<double> x) {
-  return mk<double>(__shfl_xor(x.re, 32), __shfl_xor(x.im, 32));
-}
-
-// Schur-vector engine of k_qr64: this lane's half row zh[c] = Z(row, 32 h + c).
-__device__ __forceinline__ void replay_sweeps_half(const QrShared64 &sh, int h, cx<double> (&zh)[32]) {
-  int buf = 0;
-  for (;;) {
-    __syncthreads();
-    const SweepLog<double> &lg = sh.log[buf];
-    const int L = lg.L, I = lg.I;
-#pragma unroll
-    for (int K = 0; K + 1 < kN; ++K) {
-      if (K >= L && K < I) {
-        const cx<double> t1 = ld<double>(&lg.t1[K]), v2 = ld<double>(&lg.v2[K]);
-        const double t2 = t1.re * v2.re - t1.im * v2.im;
-        if (K + 1 < 32) {
-          if (h == 0) {
-            const cx<double> sum = add(mul(t1, zh[K]), scale(zh[K + 1], t2));
-            zh[K] = sub(zh[K], sum);
-            zh[K + 1] = sub(zh[K + 1], mulc(sum, v2));
-          }
-        } else if (K >= 32) {
-          if (h == 1) {
-            const cx<double> sum = add(mul(t1, zh[K - 32]), scale(zh[K - 31], t2));
-            zh[K - 32] = sub(zh[K - 32], sum);
-            zh[K - 31] = sub(zh[K - 31], mulc(sum, v2));
-          }
-        } else {
-          // columns 31 and 32: one in each half of the row
-          const cx<double> mine = h == 0 ? zh[31] : zh[0];
-          const cx<double> other = half_swap(mine);
-          const cx<double> z31 = h == 0 ? mine : other, z32 = h == 0 ? other : mine;
-          const cx<double> sum = add(mul(t1, z31), scale(z32, t2));
-          if (h == 0) zh[31] = sub(z31, sum);
-          else zh[0] = sub(z32, mulc(sum, v2));
-        }
-      }
-    }
-    if (lg.has_phase) {
-      const cx<double> ph = ld<double>(&lg.phase);
-#pragma unroll
-      for (int c = 1; c < kN; ++c)
-        if (c == I && h == c / 32) zh[c % 32] = mulc(zh[c % 32], ph);
-    }
-    const int last = lg.last;
-    buf ^= 1;
-    if (last) break;
-  }
-}
-
-typedef double d4 __attribute__((ext_vector_type(4)));
-
-// The back-transform V = Z X of ztrevc (Toolbox.hpp:1268-1275) for the 32
-// rows row0..row0+31 of Z this wavefront holds as half rows (lane l: row
-// row0 + l % 32, columns 32 (l / 32) .. +31 in zh), on the FP64 matrix
-// cores: v_mfma_f64_16x16x4f64 multiplies a 16 x 4 slice of Z (A operand:
-// lane (c, q) = (l % 16, l / 16) supplies Z(16 I + c, k0 + q)) by a 4 x 16
-// slice of X (B operand: X(k0 + q, 16 J + c), read from the tile, where the
-// solve left y = -x above the diagonal) into a 16 x 16 block of V (lane
-// (c, q), slot s: V(16 I + 4 s + q, 16 J + c)).  The complex product is four
-// real products.  The A operand's entry lives in lane 16 I + c + 32 (k0 / 32)
-// of the wavefront, register k0 % 32 + q: four lane permutes per slice (one
-// per q) and a select.  X is unit upper triangular: column block J needs the
-// row blocks K <= J only.  The result goes straight to the V planes.
-__device__ __forceinline__ void backtransform_mfma(const GBand &g, const cx<double> (&zh)[32], int row0, int lane,
-                                                   int64_t base, const FusedArgs &a) {
-  const int n = g.n;
-  const int c = lane & 15, q = lane >> 4;
-  // one 16 x 16 block of V at a time (runtime loops: Z's 32 half-row entries
-  // take most of the registers, so only one block's accumulators stay live)
-  for (int blk = 0; blk < 8; ++blk) {
-    const int I = blk & 1, J = blk >> 1;
-    if (16 * J >= n) break;  // wavefront-uniform
-    d4 vre = d4{0, 0, 0, 0}, vim = d4{0, 0, 0, 0};
-#pragma unroll
-    for (int K = 0; K < 4; ++K) {
-      if (K > J) break;  // X is upper triangular
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int k = 16 * K + 4 * s + q, j = 16 * J + c;
-        cx<double> x = mk<double>(k == j ? 1.0 : 0.0, 0);
-        if (k < j) {
-          const cx<double> y = ld<double>(g.at(k, j));
-          x = mk<double>(-y.re, -y.im);
-        }
-        const int src = 16 * I + c + 32 * (K >> 1);
-        cx<double> za = mk<double>(0, 0);
-#pragma unroll
-        for (int qq = 0; qq < 4; ++qq) {
-          const cx<double> zr = zh[16 * (K & 1) + 4 * s + qq];
-          const double re = __shfl(zr.re, src), im = __shfl(zr.im, src);
-          if (qq == q) za = mk<double>(re, im);
-        }
-        vre = __builtin_amdgcn_mfma_f64_16x16x4f64(za.re, x.re, vre, 0, 0, 0);
-        vre = __builtin_amdgcn_mfma_f64_16x16x4f64(-za.im, x.im, vre, 0, 0, 0);
-        vim = __builtin_amdgcn_mfma_f64_16x16x4f64(za.re, x.im, vim, 0, 0, 0);
-        vim = __builtin_amdgcn_mfma_f64_16x16x4f64(za.im, x.re, vim, 0, 0, 0);
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int row = row0 + 16 * I + 4 * s + q, col = 16 * J + c;
-      if (row < n && col < n) {
-        const int64_t idx = base + a.G.el(row, col);
-        a.rV[idx] = vre[s];
-        a.iV[idx] = vim[s];
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(192) __attribute__((amdgpu_waves_per_eu(3))) void k_qr64(FusedArgs a) {
-  __shared__ QrShared64 sh;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t m = xcd_block();
-  if (m >= a.G.nmat) return;  // workgroup-uniform
-  const int n = a.G.n, nmax = a.G.n;
-  const int64_t base = a.G.mat_base(m), vbase = a.G.vec_base(m);
-  GBand g;
-  g.mi = 0;
-  g.r = lane;
-  g.n = n;
-  g.H = sh.H;
-  g.vsh = nullptr;
-  if (w == 0) {
-    // the Hessenberg part of the reduction's output, into the band
-    for (int i = lane; i < GBand::kSize; i += 64) st<double>(sh.H + i, mk<double>(0, 0));
-    wave_sync();
-    if (lane < n)
-      for (int c = lane > 0 ? lane - 1 : 0; c < n; ++c) {
-        const int64_t idx = base + a.G.el(lane, c);
-        st<double>(g.at(lane, c), mk<double>(a.rV[idx], a.iV[idx]));
-      }
-  }
-  __syncthreads();
-  if (w == 0) {
-    // ---------------- Hessenberg engine ----------------
-    const int nfail = lahqr_recorded(g, sh, a.itmax);
-    if (a.flags & VEIG_WRITE_SCHUR) {
-      if (lane < n)
-        for (int c = 0; c < n; ++c) {
-          const int64_t idx = base + a.G.el(lane, c);
-          const cx<double> t = c >= lane ? ld<double>(g.at(lane, c)) : mk<double>(0, 0);
-          a.rA[idx] = t.re;
-          a.iA[idx] = t.im;
-        }
-    }
-    const cx<double> lam = trevc_solve_lds(g, nmax);  // leaves y = -x above the diagonal
-    if (lane < n) {
-      a.rE[vbase + a.G.ve(lane)] = lam.re;
-      a.iE[vbase + a.G.ve(lane)] = lam.im;
-    }
-    if (a.info && lane == 0) a.info[m] = nfail;
-    __syncthreads();  // the eigenvector factor is ready
-  } else {
-    // ---------------- Schur-vector engines: half a row per lane ----------------
-    const int h = lane >> 5;
-    const int row = (w - 1) * 32 + (lane & 31);
-    cx<double> zh[32];
-#pragma unroll
-    for (int c = 0; c < 32; ++c) zh[c] = mk<double>(32 * h + c == row ? 1.0 : 0.0, 0);
-    // Q = H_0 H_1 ... H_{n-2} from the reflectors the reduction left in V and
-    // E: lane l loads v(l) of reflector i, and each lane fetches the 32
-    // entries of its half row from the other lanes (a lane permute, no LDS),
-    // once for w = Z v and again for the update Z -= tau w v^H
-    for (int i = 0; i + 1 < nmax; ++i) {
-      cx<double> vl = mk<double>(lane == i + 1 ? 1.0 : 0.0, 0);
-      if (lane >= i + 2 && lane < n) {
-        const int64_t idx = base + a.G.el(lane, i);
-        vl = mk<double>(a.rV[idx], a.iV[idx]);
-      }
-      const cx<double> tau = mk<double>(a.rE[vbase + a.G.ve(i)], a.iE[vbase + a.G.ve(i)]);
-      int src = 32 * h;
-      asm volatile("" : "+v"(src));
-      cx<double> wv = mk<double>(0, 0);
-#pragma unroll
-      for (int c = 0; c < 32; ++c)
-        wv = add(wv, mul(zh[c], mk<double>(__shfl(vl.re, src + c), __shfl(vl.im, src + c))));
-      wv = add(wv, half_swap(wv));
-      const cx<double> tw = mul(tau, wv);
-      asm volatile("" : "+v"(src));  // permute again rather than keep 32 values live
-#pragma unroll
-      for (int c = 0; c < 32; ++c)
-        zh[c] = sub(zh[c], mulc(tw, mk<double>(__shfl(vl.re, src + c), __shfl(vl.im, src + c))));
-    }
-    replay_sweeps_half(sh, h, zh);
-    __syncthreads();  // the eigenvector factor is ready
-    backtransform_mfma(g, zh, (w - 1) * 32, lane, base, a);
-  }
+  solve_one<float, OUT>(a, sh, m, w, lane);
 }
 
 }  // namespace
 
 namespace veig {
-template <typename R, int OUT>
+template <int OUT>
 int launch_zgeev64(const FusedArgs &a, hipStream_t s) {
-  if (a.G.nmat > INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
-  if (a.mask) return fail(VEIG_ERR_UNSUPPORTED, "orders above 32: no masked launches");
-  if (a.list) {
-    // the FP64 solve of the matrices the mixed path hands back
-    if constexpr (std::is_same<R, double>::value && OUT == OUT_V) {
-      const int64_t g = a.G.nmat < kListGrid ? a.G.nmat : kListGrid;
-      hipLaunchKernelGGL((k_zgeev64_list<R, OUT>), dim3((unsigned)g), dim3(128), 0, s, a);
-    } else {
-      return fail(VEIG_ERR_UNSUPPORTED, "orders above 32: list launches are FP64 only");
-    }
-  } else if constexpr (std::is_same<R, double>::value && OUT == OUT_V) {
-    hipLaunchKernelGGL(k_gehrd64, dim3((unsigned)a.G.nmat), dim3(64 * reduce_waves<kN>()), 0, s, a);
-    hipLaunchKernelGGL(k_qr64, dim3((unsigned)a.G.nmat), dim3(192), 0, s, a);
-  } else {
-    hipLaunchKernelGGL((k_zgeev64<R, OUT>), dim3((unsigned)a.G.nmat), dim3(128), 0, s, a);
-  }
+  if (a.mask || a.list) return fail(VEIG_ERR_UNSUPPORTED, "complex64 above order 32: whole batches only");
+  hipLaunchKernelGGL((k_zgeev64<OUT>), dim3((unsigned)a.G.nmat), dim3(128), 0, s, a);
   VEIG_HIP(hipGetLastError());
   return VEIG_OK;
 }
-template int launch_zgeev64<double, OUT_V>(const FusedArgs &, hipStream_t);
-template int launch_zgeev64<float, OUT_V>(const FusedArgs &, hipStream_t);
-template int launch_zgeev64<float, OUT_VW>(const FusedArgs &, hipStream_t);
+template int launch_zgeev64<OUT_V>(const FusedArgs &, hipStream_t);
+template int launch_zgeev64<OUT_VW>(const FusedArgs &, hipStream_t);
 }  // namespace veig

@@ -20,7 +20,7 @@
 #include <cstdint>
 #include <string>
 
-#include "veig_common.hpp"
+#include "veig_stream.hpp"
 
 using namespace veig;
 
@@ -60,6 +60,15 @@ __device__ __forceinline__ void companion_rows(const G &g, const EigArgs &a, int
     }
   }
 }
+
+// what companion_rows asks of one matrix per wavefront on a BandTile
+struct BandRows {
+  static constexpr int LG = 64, LD = 65;
+  BandTile t;
+  int n, lane;
+  __device__ __forceinline__ int idx(int p) const { return lane + 64 * p; }
+  __device__ __forceinline__ double2 *at(int r, int c) const { return t.at(r, c); }
+};
 
 // LDS of a wavefront's MPW matrices in layout LAY, and each group's vector:
 // the reflector of the Hessenberg reduction (dense layout), or just the two
@@ -152,6 +161,93 @@ __global__ __launch_bounds__(64) void k_eig(EigArgs a) {
   if (a.info && valid && g.r == 0) a.info[m] = nfail;
 }
 
+// Orders 33..64, eigenvalues only: the reduction by the whole workgroup on a
+// dense tile, then the iteration by its first wavefront in the same tile
+// (lahqr_stream; the others are done).  Order 48 x 16,384: 23.6 ms, against
+// 60.7 ms for one wavefront doing both on a 66 KB tile; at 41 KB four
+// workgroups share a CU, one chain per SIMD, and the chain's issue rate bounds
+// them (see lahqr_stream).
+template <int CAP, int W>
+__global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_eig_block(EigArgs a) {
+  using S = ReduceBlock<CAP, W>;
+  extern __shared__ double2 lds[];
+  S &sm = *reinterpret_cast<S *>(lds);
+  const int64_t m = xcd_block();
+  if (m >= a.G.nmat) return;  // workgroup-uniform
+  const int n = a.G.n;
+  reduce_load(sm, n, a.G, a.G.mat_base(m), a.rA, a.iA);
+  reduce_block(sm, n, nullptr);
+  const int lane = threadIdx.x & 63;
+  const DenseTile<S::LD> t{sm.H};
+  auto &rec = *reinterpret_cast<SweepScratch<CAP> *>(sm.part);  // free now
+  static_assert(sizeof(rec) <= sizeof(sm.part), "the record fits the reduction's partial sums");
+  if ((int)(threadIdx.x >> 6) == chain_wave(rec.simd)) {
+    const int nfail = lahqr_stream<1, false>(t, n, lane, rec, a.itmax);
+    const int64_t vb = a.G.vec_base(m);
+    if (lane < n) {
+      const cx<double> e = ld<double>(t.at(lane, lane));
+      a.rE[vb + a.G.ve(lane)] = e.re;
+      a.iE[vb + a.G.ve(lane)] = e.im;
+    }
+    if (a.info && lane == 0) a.info[m] = nfail;
+  }
+  __syncthreads();  // the idle wavefronts keep their places (chain_wave) until the end
+}
+
+// Orders 33..64 that start from a Hessenberg matrix: one wavefront per matrix
+// on the banded tile
+template <int SRC>
+__global__ __launch_bounds__(64) void k_eig_band(EigArgs a) {
+  extern __shared__ double2 lds[];
+  __shared__ SweepScratch<64> rec;
+  const int64_t m = xcd_block();
+  if (m >= a.G.nmat) return;
+  const int n = a.G.n, lane = threadIdx.x;
+  const BandTile t{lds};
+  for (int i = lane; i < BandTile::entries(n); i += 64) st<double>(lds + i, mk<double>(0, 0));
+  lds_order();
+  const int64_t base = a.G.mat_base(m), vb = a.G.vec_base(m);
+  if constexpr (SRC == SRC_POLY) {
+    BandRows g{t, n, lane};
+    companion_rows(g, a, m);
+  } else {
+    for (int c = 0; c < n; ++c)
+      if (lane <= c + 1 && lane < n) {
+        const int64_t idx = base + a.G.el(lane, c);
+        st<double>(t.at(lane, c), mk<double>(a.rA[idx], a.iA[idx]));
+      }
+  }
+  lds_order();
+  const int nfail = lahqr_stream<1, false>(t, n, lane, rec, a.itmax);
+  if (lane < n) {
+    const cx<double> e = ld<double>(t.at(lane, lane));
+    a.rE[vb + a.G.ve(lane)] = e.re;
+    a.iE[vb + a.G.ve(lane)] = e.im;
+  }
+  if constexpr (SRC == SRC_HESSENBERG) {
+    // the Hessenberg part back (entries below the subdiagonal untouched)
+    for (int c = 0; c < n; ++c)
+      if (lane <= c + 1 && lane < n) {
+        const int64_t idx = base + a.G.el(lane, c);
+        const cx<double> h = ld<double>(t.at(lane, c));
+        a.rH[idx] = h.re;
+        a.iH[idx] = h.im;
+      }
+  }
+  if (a.info && lane == 0) a.info[m] = nfail;
+}
+
+template <int CAP, int W>
+int launch_eig_block(const EigArgs &a, hipStream_t s) {
+  using S = ReduceBlock<CAP, W>;
+  if (sizeof(S) > 64 * 1024)
+    VEIG_HIP(hipFuncSetAttribute((const void *)k_eig_block<CAP, W>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)sizeof(S)));
+  hipLaunchKernelGGL((k_eig_block<CAP, W>), dim3((unsigned)a.G.nmat), dim3(S::kThreads), sizeof(S), s, a);
+  VEIG_HIP(hipGetLastError());
+  return VEIG_OK;
+}
+
 template <int SRC, bool TZ>
 int launch_eig(const EigArgs &a, hipStream_t s) {
   if (a.G.nmat > (int64_t)INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
@@ -162,7 +258,16 @@ int launch_eig(const EigArgs &a, hipStream_t s) {
     case 8: hipLaunchKernelGGL((k_eig<8, 1, SRC, TZ>), dim3(grid), dim3(64), 0, s, a); break;
     case 16: hipLaunchKernelGGL((k_eig<16, 1, SRC, TZ>), dim3(grid), dim3(64), 0, s, a); break;
     case 32: hipLaunchKernelGGL((k_eig<32, 1, SRC, TZ>), dim3(grid), dim3(64), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_eig<64, 1, SRC, TZ>), dim3(grid), dim3(64), 0, s, a); break;
+    default:
+      if constexpr (SRC == SRC_MATRIX) {
+        return a.G.n <= 48 ? launch_eig_block<48, 4>(a, s) : launch_eig_block<64, 4>(a, s);
+      } else if constexpr (TZ) {
+        return launch_big(BIG_ROOTS, a.G, a.rH, a.iH, a.rZ, a.iZ, a.rE, a.iE, a.info, a.itmax, 0, s, nullptr, nullptr,
+                          a.rA, a.iA);
+      } else {
+        const size_t bytes = (size_t)BandTile::entries(a.G.n) * sizeof(double2);
+        hipLaunchKernelGGL((k_eig_band<SRC>), dim3(grid), dim3(64), bytes, s, a);
+      }
   }
   VEIG_HIP(hipGetLastError());
   return VEIG_OK;
