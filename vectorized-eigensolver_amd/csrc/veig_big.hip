@@ -22,13 +22,13 @@
 // order 79 x 3,328: 51 -> 34 ms, whose two workgroups of six wavefronts do not
 // share a CU at three), at 32 columns to three.
 //
-// Measured (both kernels; in brackets the kernels these replaced, whose bulge
-// chase went through LDS): order 64 x 65,536 194 ms (368), order 79 x 3,328
-// 38 ms (233: a workgroup barrier per half step and Z in global memory), the
-// stages hessenberg + zlahqr + ztrevc at order 40 x 2,048 3.2 ms (21).  What
-// bounds order 64 now is the chain wavefront's instruction issue: 7,700 steps
-// of 600 cycles and 230 sweeps of 2,400 more are 2.2 of the 2.3 ms that four
-// matrices take on a CU.
+// Measured, whole passes (in brackets the kernels these replaced, whose bulge
+// chase went through LDS): order 64 x 65,536 181 ms (371), order 79 x 3,328
+// 36 ms (233: a workgroup barrier per half step and Z in global memory), the
+// stages hessenberg + zlahqr + ztrevc at order 40 x 2,048 3.1 ms (21).  What
+// bounds order 64 is instruction issue, the chain wavefront's (7,700 steps of
+// about 88 instructions and 230 sweeps of about 480 more per matrix) and,
+// on the same SIMDs, the Schur vectors'.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>

@@ -280,7 +280,7 @@ __device__ __forceinline__ void form_q_block(ReduceBlock<CAP, W> &sm, int n, con
 // --------------------------------------------------------------------------
 // A ring of R sweeps of rotations for steps 0..CAP-1; a step outside its
 // sweep holds the identity, so the Schur-vector wavefronts apply every entry
-// without asking.  Entry K: (Re c, Im c) and (s, r), r the step's new H(K, K-1)
+// without asking.  Entry K: (Re c, Im c) and (s, r^2), r the step's new H(K, K-1)
 // (the iteration's own use).
 struct StepRec {
   double2 c, sr;
@@ -290,19 +290,17 @@ struct SweepRing {
   static constexpr int CAP = CAP_, R = R_;
   static constexpr bool kReplayed = true;
   StepRec step[R][CAP];
-  double2 trash;   // where lanes outside an update store
   double2 ph[R];   // conj(h/|h|) of the sweep's last step: column I is scaled by its conjugate
   int L[R], I[R];  // steps L..I-1
   int last[R];
   int simd[8];     // chain_wave
 };
-// the record of a wavefront that keeps no Schur vectors: this sweep's r only
+// the record of a wavefront that keeps no Schur vectors: this sweep's r^2 only
 template <int CAP_>
 struct SweepScratch {
   static constexpr int CAP = CAP_, R = 1;
   static constexpr bool kReplayed = false;
   StepRec step[1][CAP];
-  double2 trash;
   int simd[4];
 };
 
@@ -371,97 +369,106 @@ __device__ __forceinline__ void make_subdiag_real(const T &t, int n, int lane, d
 // the iteration cap.
 //
 // A wavefront alone issues one instruction per 5 cycles, so the step's
-// instruction count is its time: the 64 FP64 instructions it cannot do without
-// (the rotation 13, the window 27, the column and row updates 12 each) and as
-// few others as possible.  Hence: stores without execution masks (a lane
-// outside an update stores to `trash`, lanes past the order repeat the last
-// column), record entries written by every lane, running addresses.
+// instruction count is its time: the 51 FP64 instructions it cannot do without
+// (the rotation 12, the window 27, the update of rows and columns 12) and as
+// few others as possible.  Hence: one update for the lanes ahead of the bulge
+// and behind it, stores without execution masks (lanes past the order repeat
+// the last column), record entries written by every lane, running addresses.
 // --------------------------------------------------------------------------
 struct StreamWindow {
   cx<double> a0;   // H(K, K-1): the rotation's input
   double a1;       // H(K+1, K-1), real
+  double m2;       // |a0|^2 + a1^2
   cx<double> x1;   // H(K, K)
   cx<double> x2;   // H(K+1, K)
   double hs;       // H(K+2, K+1), real, not yet rotated
+  uint64_t none, none_hi;  // bit K (K - 64): step K's input was zero, its rotation the identity
+  cx<double> was;       // a0 where the last one was replaced
+
+  // m2, and the zero vector (or one below the underflow threshold) replaced
+  // by one that gives G = I
+  __device__ __forceinline__ void norm(int K) {
+    m2 = fma(a0.re, a0.re, fma(a0.im, a0.im, a1 * a1));
+    if (__builtin_expect(__any(m2 == 0.0), 0)) {
+      was = a0;
+      a0 = mk<double>(1, 0);
+      a1 = 0.0;
+      m2 = 1.0;
+      const uint64_t bit = 1ull << (K & 63);
+      none |= K < 64 ? bit : 0;
+      none_hi |= K < 64 ? 0 : bit;
+    }
+  }
 };
 
-// the running state of a sweep: entry of row lane (+ 64) in column K and of
-// column lane (+ 64) in row K, the operands that the next step rotates them
-// with, and the addresses (LDS, in entries) of what the step stores and loads
+// The running state of a sweep.  Lane t is ahead of the bulge (t > K) or behind
+// it (t < K), and the two updates it then takes part in are the same one but
+// for the sign of Im c (rot_left by q is rot_right by its conjugate): ahead,
+// rows K, K+1 of column t by this step's rotation; behind, columns K-1, K of
+// row t by the last one's (these lag by a step, so that row K has its entry
+// of column K+1).  So one update serves both, 12 FP64 instructions and one
+// store and load per lane, and a lane changes its role as the bulge passes it.
+// (Each lane taking both updates at every step, half of them to no use: order
+// 64 x 65,536 198 ms instead of 181.  All lanes a step behind the
+// window, so that the update fills the latency of the reciprocal square root:
+// 191 ms, the window then having an entry more to rotate.)
 template <int P>
 struct StreamLanes {
-  cx<double> u[P], w[P], hr[P], hl[P];
-  Rot<double> qp;     // the last step's rotation (the row updates lag by one step)
-  double sd[P];       // H(lane + 2, lane + 1), real
-  double2 *pc[P];     // H(K, lane)
-  double2 *pr[P];     // H(lane, K - 1)
+  cx<double> e[P];     // the running entry: H(K, t) ahead, H(t, K-1) behind
+  cx<double> o[P];     // the entry that the next rotation pairs it with
+  Rot<double> q;       // the last step's rotation
+  double sd[P];        // H(t + 2, t + 1), real
+  double2 *pe[P], *po[P];  // their places in the tile
+  int t[P];            // this lane's row and column
 };
 
-// one step; W0: the first slot whose columns are still ahead (0, or P - 1
-// once K + 1 has passed lane 63), RP: slots whose rows have been reached
-template <int P, int W0, int RP, bool TZ, typename T>
-__device__ __forceinline__ void stream_step(int lane, int L, int I, int K, StreamWindow &x,
-                                            StreamLanes<P> &a, StepRec *rec, double2 *trash) {
+// step K; M: the slot that the bulge is passing (slots before it are behind,
+// slots after it ahead), Y: the slot of column K + 1; REC: the whole record,
+// or r^2 only
+template <int P, int M, int Y, bool REC, typename T>
+__device__ __forceinline__ void stream_step(int K, StreamWindow &x, StreamLanes<P> &a, StepRec *rec) {
   using R = double;
-  R nb0, nrm2;
-  Rot<R> q = rot2(x.a0, x.a1, nb0, nrm2);
-  if (__builtin_expect(__any(nrm2 == 0.0), 0)) {  // the zero vector: G = I
-    q.c = mk<R>(1, 0);
-    q.s = 0.0;
-    nb0 = 0.0;
+  const R m2 = x.m2, ir = frsq(m2);
+  const Rot<R> q{mk(x.a0.re * ir, x.a0.im * ir), x.a1 * ir};
+  if constexpr (REC) {
+    rec[K].c = double2{q.c.re, q.c.im};
+    rec[K].sr = double2{q.s, m2};
+  } else {
+    rec[K].sr.y = m2;
   }
-  // columns K-1, K over rows 0..K-1: the last step's rotation (one step late,
-  // its operand loaded at that step's end)
-  const int wk = T::width(K - 1), wk1 = T::width(K);
+  const int wk = T::width(K);
+  bool ahead[P];
 #pragma unroll
-  for (int p = 0; p < RP; ++p) {
-    cx<R> o = a.u[p];
-    rot_right(a.qp, o, a.hr[p]);
-    a.u[p] = a.hr[p];
-    const int row = lane + 64 * p;
-    double2 *d = row < K ? a.pr[p] : trash;
-    if constexpr (!TZ) d = row >= L ? d : trash;
-    st<R>(d, o);
-    a.pr[p] += wk;
+  for (int p = 0; p < P; ++p) {
+    ahead[p] = p > M || (p == M && a.t[p] > K);
+    const Rot<R> g{mk(ahead[p] ? q.c.re : a.q.c.re, ahead[p] ? -q.c.im : a.q.c.im), ahead[p] ? q.s : a.q.s};
+    cx<R> out = a.e[p];
+    rot_right(g, out, a.o[p]);
+    a.e[p] = a.o[p];
+    st<R>(a.pe[p], out);  // (lane K: overwritten by itself at the next step)
   }
-  rec[K].c = double2{q.c.re, q.c.im};
-  rec[K].sr = double2{q.s, nb0};
-  // rows K, K+1 over columns K+1..n-1
-#pragma unroll
-  for (int p = W0; p < P; ++p) {
-    cx<R> o = a.w[p];
-    rot_left(q, o, a.hl[p]);
-    a.w[p] = a.hl[p];
-    const int col = lane + 64 * p;
-    double2 *d = col > K ? a.pc[p] : trash;
-    if constexpr (!TZ) d = col <= I ? d : trash;
-    st<R>(d, o);
-  }
-  // the window: column K of rows K, K+1, then rows K, K+1 of columns K, K+1
+  // the window: column K of rows K, K+1, then row K+1 of columns K, K+1
   cx<R> x1 = x.x1, x2 = x.x2;
   rot_left(q, x1, x2);
   const int src = (K + 1) & 63;
-  cx<R> y2 = mk(read_lane(a.w[W0].re, src), read_lane(a.w[W0].im, src));
-#pragma unroll
-  for (int p = 0; p < RP; ++p)
-    if (lane + 64 * p == K) a.u[p] = x1;  // row K enters the row updates
+  cx<R> y2 = mk(read_lane(a.e[Y].re, src), read_lane(a.e[Y].im, src));
   rot_right(q, x2, y2);
   x.a0 = x2;
   x.x1 = y2;
   x.a1 = q.s * x.hs;
+  x.norm(K + 1);
   x.x2 = mk(q.c.re * x.hs, -q.c.im * x.hs);
-  a.qp = q;
-  // operands of the next step's updates (past the last row and column: read
-  // and not used)
+  x.hs = read_lane(a.sd[Y], src);
+  a.q = q;
   lds_order();
 #pragma unroll
-  for (int p = 0; p < RP; ++p) a.hr[p] = ld<R>(a.pr[p] + wk1);
-#pragma unroll
   for (int p = 0; p < P; ++p) {
-    if (p >= W0) a.hl[p] = ld<R>(a.pc[p] + 2);
-    a.pc[p] += 1;
+    const bool pass = p == M && a.t[p] == K;  // the bulge passes lane K: x1 is row K's first entry
+    a.e[p] = mk(pass ? x1.re : a.e[p].re, pass ? x1.im : a.e[p].im);
+    a.pe[p] = pass ? a.pe[p] : a.po[p];
+    a.po[p] = a.pe[p] + (ahead[p] ? 1 : wk);
+    a.o[p] = ld<R>(a.po[p]);  // past the last row and column: read and not used
   }
-  x.hs = read_lane(a.sd[W0], src);
 }
 
 template <int P, bool TZ, typename T, typename RING>
@@ -469,6 +476,7 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
   using R = double;
   constexpr bool kRec = RING::kReplayed;
   constexpr int CAP = RING::CAP, kR = RING::R;
+  static_assert(TZ || P == 1, "the active block's lanes sit in one slot");
   const R ulp = limits<R>::eps;
   const R smlnum = limits<R>::tiny * (R(n > 0 ? n : 1) / ulp);
   int rt[P];  // lanes past the order repeat its last row and column
@@ -547,26 +555,32 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
     StreamWindow x;
     x.a0 = cldexp(h11s, -E1);
     x.a1 = fldexp(h21, -E1);
+    x.none = x.none_hi = 0;
+    x.norm(L);
     x.x1 = h11;
     x.x2 = mk<R>(h21, 0.0);
     x.hs = t.at(L + 2, L + 1)->x;  // past the last row: read and not used
 
     // ---- the sweep (Toolbox.hpp:138-335) ----
-    // a step "L - 1" by the identity brings column L into the row updates
-    // and rewrites column L - 1 unchanged (L = 0: to the trash)
+    // the identity as the rotation before the first brings column L into the
+    // row updates and rewrites column L - 1 unchanged
     StreamLanes<P> a;
-    a.qp = Rot<R>{mk<R>(1, 0), 0.0};
-    double2 *trash = &ring.trash;
+    a.q = Rot<R>{mk<R>(1, 0), 0.0};
     StepRec *rec = ring.step[slot];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-      a.u[p] = ld<R>(t.at(rt[p], L > 0 ? L - 1 : 0));
-      a.hr[p] = ld<R>(t.at(rt[p], L));
-      a.pc[p] = t.at(L, rt[p]);
-      a.pr[p] = t.at(rt[p], L) - T::width(L - 1);
-      a.w[p] = ld<R>(a.pc[p]);
-      a.hl[p] = ld<R>(a.pc[p] + 1);
-      const int sc = lane + 64 * p + 1 < I ? lane + 64 * p + 1 : I - 1;
+      // lanes past the order repeat the last column, always ahead; without
+      // the Schur form the lanes outside the active block repeat column I
+      const int t0 = lane + 64 * p;
+      const bool in = TZ || (t0 >= L && t0 <= I);
+      const int at = in ? rt[p] : I;
+      a.t[p] = in ? t0 : I;
+      const bool behind = a.t[p] < L;
+      a.po[p] = behind ? t.at(at, L) : t.at(L, at) + 1;
+      a.pe[p] = a.po[p] - (behind ? T::width(L - 1) : 1);
+      a.e[p] = ld<R>(a.pe[p]);
+      a.o[p] = ld<R>(a.po[p]);
+      const int sc = t0 + 1 < I ? t0 + 1 : I - 1;
       a.sd[p] = t.at(sc + 1, sc)->x;
     }
     if constexpr (kRec) {
@@ -576,33 +590,34 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
     // (two steps per turn: the state alternates between two sets of registers
     // instead of being copied)
     int K = L;
-    auto run = [&](auto w0, auto rp, int end) {
-      constexpr int W0 = decltype(w0)::value, RP = decltype(rp)::value;
+    auto run = [&](auto mc, auto yc, int end) {
+      constexpr int M = decltype(mc)::value, Y = decltype(yc)::value;
       for (; K + 1 < end; K += 2) {
-        stream_step<P, W0, RP, TZ, T>(lane, L, I, K, x, a, rec, trash);
-        stream_step<P, W0, RP, TZ, T>(lane, L, I, K + 1, x, a, rec, trash);
+        stream_step<P, M, Y, kRec, T>(K, x, a, rec);
+        stream_step<P, M, Y, kRec, T>(K + 1, x, a, rec);
       }
       if (K < end) {
-        stream_step<P, W0, RP, TZ, T>(lane, L, I, K, x, a, rec, trash);
+        stream_step<P, M, Y, kRec, T>(K, x, a, rec);
         ++K;
       }
     };
-    using std::integral_constant;
+    constexpr std::integral_constant<int, 0> s0;
+    constexpr std::integral_constant<int, P - 1> s1;
     if constexpr (P == 1) {
-      run(integral_constant<int, 0>{}, integral_constant<int, 1>{}, I);
+      run(s0, s0, I);
     } else {
-      // columns up to 63 still ahead; then rows from 63 on reached
-      run(integral_constant<int, 0>{}, integral_constant<int, 1>{}, I < 63 ? I : 63);
-      if (K < I) {
-        a.pr[P - 1] = t.at(rt[P - 1], K) - T::width(K - 1);
-        a.hr[P - 1] = mk<R>(0, 0);
-        run(integral_constant<int, P - 1>{}, integral_constant<int, P>{}, I);
+      // column K + 1 in the first slot, then row K (K = 63) in the first slot
+      run(s0, s0, I < 63 ? I : 63);
+      if (K == 63 && I > 63) {
+        stream_step<P, 0, P - 1, kRec, T>(K, x, a, rec);
+        ++K;
       }
+      if (K < I) run(s1, s1, I);
     }
     // the last rotation's rows, then H(I, I-1) made real (Toolbox.hpp:337-367)
     // on the way out: row I right of I and column I above it scaled
     cx<R> zz = mk<R>(1, 0);
-    cx<R> hsub = x.a0;
+    cx<R> hsub = ((I < 64 ? x.none : x.none_hi) >> (I & 63)) & 1u ? x.was : x.a0;
     if (hsub.im != 0.0 && abs2(hsub) > 0.0) {  // |h|^2 may underflow: leave such h alone
       const R m2 = abs2(hsub), id = frsq(m2);
       zz = mk(hsub.re * id, -hsub.im * id);  // conj(h/|h|)
@@ -612,14 +627,17 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int q = lane + 64 * p;
-      cx<R> o = a.u[p], c = a.hr[p];
-      rot_right(a.qp, o, c);
+      cx<R> o = a.e[p], c = a.o[p];
+      rot_right(a.q, o, c);
       if (q < I && (TZ || q >= L)) {
         st<R>(t.at(rt[p], I - 1), o);
         st<R>(t.at(rt[p], I), mulc(c, zz));
       }
-      if (TZ && q > I && q < n) st<R>(t.at(I, rt[p]), mul(a.w[p], zz));
-      if (q > L && q < I) st<R>(t.at(q, q - 1), mk<R>(rec[q].sr.y, 0.0));
+      if (TZ && q > I && q < n) st<R>(t.at(I, rt[p]), mul(a.e[p], zz));
+      if (q > L && q < I) {  // H(q, q-1) = r
+        const R m2 = rec[q].sr.y, r = m2 * frsq(m2);
+        st<R>(t.at(q, q - 1), mk<R>(((p == 0 ? x.none : x.none_hi) >> lane) & 1u ? 0.0 : r, 0.0));
+      }
     }
     if (lane == 0) {
       st<R>(t.at(I, I - 1), hsub);
