@@ -38,6 +38,21 @@ struct StageArgs {
 
 enum { ST_GEHRD = 0, ST_HESS = 1, ST_UNGHR = 2, ST_LAHQR = 3, ST_TREVC = 4 };
 
+// Whether a stage entry runs one matrix per workgroup (veig_big.hip) rather
+// than on lane groups.  Above order 16 the reduction, zunghr and ztrevc always
+// do: the lane groups' dense tiles leave one wavefront per SIMD there
+// (65,536 matrices, lane groups -> workgroups: hessenberg of order 17 2.58 ->
+// 2.25 ms, 24 4.42 -> 3.01, 32 7.03 -> 4.00; ztrevc 1.11 -> 0.95, 1.92 -> 1.49,
+// 2.88 -> 2.27; at order 16 they lose, 0.65 -> 0.71 and 0.33 -> 0.73).  Below
+// it the reduction does up to four matrices per CU (order 16 x 1,024: 68 ->
+// 44 us), the QR iteration up to one (few_matrices).
+bool per_workgroup(int mode, const Geom &G) {
+  if (G.n > 32) return true;
+  if (mode == ST_LAHQR) return G.n >= 8 && few_matrices(G, 1);
+  if (G.n > 16) return true;
+  return mode != ST_TREVC && G.n >= 8 && few_matrices(G, 4);
+}
+
 template <int NB>
 __global__ __launch_bounds__(64) void k_stage(StageArgs a) {
   using R = double;
@@ -52,7 +67,8 @@ __global__ __launch_bounds__(64) void k_stage(StageArgs a) {
   const int nmax = a.G.n;
   wave_sync();
   cx<R> z[1][NB];
-  if (a.mode == ST_GEHRD || a.mode == ST_HESS) {
+  // (above order 16: the QR iteration only, see per_workgroup)
+  if (NB <= 16 && (a.mode == ST_GEHRD || a.mode == ST_HESS)) {
     load_rows<R, NB>(g, a.G, base, a.rA, a.iA, NB);
     identity_rows<R, NB>(g, z);
     wave_sync();
@@ -64,7 +80,7 @@ __global__ __launch_bounds__(64) void k_stage(StageArgs a) {
       a.iE[vbase + a.G.ve(g.r)] = tau.im;
     }
     if (a.mode == ST_HESS) store_row_regs<R, NB>(g, a.G, base, a.rB, a.iB, z);
-  } else if (a.mode == ST_UNGHR) {
+  } else if (NB <= 16 && a.mode == ST_UNGHR) {
     // reflector i: v = e_{i+1} + A(i+2:n, i), tau(i); Q = H_0 H_1 ... H_{n-2}
     load_rows<R, NB>(g, a.G, base, a.rA, a.iA, NB);
     identity_rows<R, NB>(g, z);
@@ -90,7 +106,7 @@ __global__ __launch_bounds__(64) void k_stage(StageArgs a) {
       for (int c = 0; c < NB; ++c) z[0][c] = sub(z[0][c], mulc(tw, ld<R>(g.vsh + c)));
     }
     store_row_regs<R, NB>(g, a.G, base, a.rA, a.iA, z);
-  } else if (a.mode == ST_LAHQR) {
+  } else if (NB > 16 || a.mode == ST_LAHQR) {
     load_rows<R, NB>(g, a.G, base, a.rA, a.iA, 1);  // Hessenberg part only
     load_row_regs<R, NB>(g, a.G, base, a.rB, a.iB, z);
     wave_sync();
@@ -299,7 +315,7 @@ int veig_zgehrd(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rA, 
   if (empty_batch(dim, block_cnt, thread_cnt)) return VEIG_OK;
   VEIG_REQUIRE(rA); VEIG_REQUIRE(iA); VEIG_REQUIRE(rtau); VEIG_REQUIRE(itau);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
-  if (dim > 32) return launch_big(BIG_GEHRD, G, rA, iA, nullptr, nullptr, rtau, itau, nullptr, 30, 0, (hipStream_t)stream);
+  if (per_workgroup(ST_GEHRD, G)) return launch_big(BIG_GEHRD, G, rA, iA, nullptr, nullptr, rtau, itau, nullptr, 30, 0, (hipStream_t)stream);
   StageArgs a{rA, iA, nullptr, nullptr, rtau, itau, nullptr, G, 30, ST_GEHRD};
   return launch_stage(a, (hipStream_t)stream);
 }
@@ -312,7 +328,7 @@ int veig_hessenberg(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *
   // tau is produced and consumed on chip (Q is accumulated forward), so no
   // tau planes are needed: the kernels skip writing it
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
-  if (dim > 32) return launch_big(BIG_HESS, G, rA, iA, rQ, iQ, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
+  if (per_workgroup(ST_HESS, G)) return launch_big(BIG_HESS, G, rA, iA, rQ, iQ, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
   StageArgs a{rA, iA, rQ, iQ, nullptr, nullptr, nullptr, G, 30, ST_HESS};
   return launch_stage(a, (hipStream_t)stream);
 }
@@ -324,7 +340,7 @@ int veig_zunghr(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rA, 
   VEIG_REQUIRE(rA); VEIG_REQUIRE(iA); VEIG_REQUIRE(rtau); VEIG_REQUIRE(itau);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
   double *rt = const_cast<double *>(rtau), *it = const_cast<double *>(itau);
-  if (dim > 32) return launch_big(BIG_UNGHR, G, rA, iA, nullptr, nullptr, rt, it, nullptr, 30, 0, (hipStream_t)stream);
+  if (per_workgroup(ST_UNGHR, G)) return launch_big(BIG_UNGHR, G, rA, iA, nullptr, nullptr, rt, it, nullptr, 30, 0, (hipStream_t)stream);
   StageArgs a{rA, iA, nullptr, nullptr, rt, it, nullptr, G, 30, ST_UNGHR};
   return launch_stage(a, (hipStream_t)stream);
 }
@@ -337,7 +353,7 @@ int veig_zlahqr(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rE, 
   VEIG_REQUIRE(rE); VEIG_REQUIRE(iE); VEIG_REQUIRE(rH); VEIG_REQUIRE(iH); VEIG_REQUIRE(rZ); VEIG_REQUIRE(iZ);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
   const int its = itmax > 0 ? itmax : 30;
-  if (dim > 32) return launch_big(BIG_LAHQR, G, rH, iH, rZ, iZ, rE, iE, info, its, 0, (hipStream_t)stream);
+  if (per_workgroup(ST_LAHQR, G)) return launch_big(BIG_LAHQR, G, rH, iH, rZ, iZ, rE, iE, info, its, 0, (hipStream_t)stream);
   StageArgs a{rH, iH, rZ, iZ, rE, iE, info, G, its, ST_LAHQR};
   return launch_stage(a, (hipStream_t)stream);
 }
@@ -349,7 +365,7 @@ int veig_ztrevc(int64_t dim, int64_t block_cnt, int64_t thread_cnt, const double
   VEIG_REQUIRE(rT); VEIG_REQUIRE(iT); VEIG_REQUIRE(rR); VEIG_REQUIRE(iR);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
   double *rt = const_cast<double *>(rT), *it = const_cast<double *>(iT);
-  if (dim > 32) return launch_big(BIG_TREVC, G, rt, it, rR, iR, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
+  if (per_workgroup(ST_TREVC, G)) return launch_big(BIG_TREVC, G, rt, it, rR, iR, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
   StageArgs a{rt, it, rR, iR, nullptr, nullptr, nullptr, G, 30, ST_TREVC};
   return launch_stage(a, (hipStream_t)stream);
 }

@@ -1,5 +1,6 @@
-// FP64 orders 33..96: the fused eigendecomposition of whole batches and lists,
-// the stage entries, and the roots entry's Schur form.
+// FP64, one matrix per workgroup: orders 33..96, the fused eigendecomposition of
+// whole batches and lists, the stage entries, and the roots entry's Schur form;
+// and the orders below where this beats the lane groups (few_matrices).
 //
 // One matrix per workgroup, two kernels:
 //
@@ -246,6 +247,8 @@ int launch_reduce(const BigArgs &a, hipStream_t s) {
 
 template <int MODE>
 int reduce_for(const BigArgs &a, hipStream_t s) {
+  if (a.G.n <= 16) return launch_reduce<16, 4, MODE>(a, s);
+  if (a.G.n <= 32) return launch_reduce<32, 4, MODE>(a, s);
   if (a.G.n <= 48) return launch_reduce<48, 4, MODE>(a, s);
   if (a.G.n <= 64) return launch_reduce<64, 4, MODE>(a, s);
   if (a.G.n <= 80) return launch_reduce<80, 8, MODE>(a, s);
@@ -266,6 +269,7 @@ int launch_schur(const BigArgs &a, hipStream_t s) {
 
 template <int MODE>
 int schur_for(const BigArgs &a, hipStream_t s) {
+  if (a.G.n <= 32) return launch_schur<16, 2, MODE>(a, s);
   if (a.G.n <= 40) return launch_schur<20, 2, MODE>(a, s);
   if (a.G.n <= 48) return launch_schur<24, 2, MODE>(a, s);
   if (a.G.n <= 64) return launch_schur<32, 2, MODE>(a, s);

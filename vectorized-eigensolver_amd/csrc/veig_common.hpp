@@ -404,6 +404,28 @@ int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, doub
                int32_t *info, int itmax, uint32_t flags, hipStream_t s, const int32_t *list = nullptr,
                const int32_t *list_count = nullptr, const double *rC = nullptr, const double *iC = nullptr);
 
+// Batches too small to fill the chip with lane groups go to the
+// one-matrix-per-workgroup kernels (veig_stream.hpp), whose single matrix is
+// done sooner: the bulge chain runs in registers (about 450 cycles a step
+// against 600 to 1,000 through LDS), the Schur vectors beside it on another
+// wavefront.  A lane-group wavefront takes 2 to 8 matrices in that time and
+// three share a SIMD, so the lane groups win as soon as the workgroups share
+// CUs.  per_cu: where the line lies, in matrices per CU; measured, one call,
+// us, lane groups -> workgroups, at 64 / 256 / 512 / 1,024 / 4,096 matrices:
+//   zgeev, order 8      114->99   115->100  114->118  120->129   128->310
+//   zgeev, order 16     299->244  299->241  299->311  309->338   352->883
+//   zgeev, order 24     568->439  568->447  589->627  637->648   916->1812
+//   zgeev, order 32     978->694  984->712  983->973  1091->1020 1593->2933
+//   zlahqr, order 16    265->226  270->223  266->283  274->302   316->753
+//   eigvals, order 16   266->201  269->197  266->209  273->215   323->491
+//   eigvals, order 32   840->578  854->586  860->863  901->897   1986->2501
+//   roots, order 16     226->181  226->179  234->193  240->194   283->454
+//   roots, order 32     692->523  677->517  693->553  735->564   1061->1968
+// so one per CU with Schur vectors, four without (eigvals above order 16: one,
+// its dense tile letting fewer workgroups share a CU).
+constexpr int64_t kComputeUnits = 256;  // MI355X
+inline bool few_matrices(const Geom &G, int per_cu) { return G.nmat <= per_cu * kComputeUnits; }
+
 // FP64 batches and lists of orders up to NB on lane groups of LW lanes
 // (0: NB): Hessenberg reduction, then the QR iteration and eigenvectors on
 // a banded tile (two kernels)
@@ -418,7 +440,7 @@ int launch_zgeev(const FusedArgs &a, hipStream_t s) {
   constexpr bool f32 = std::is_same<R, float>::value;
   if (a.G.nmat > (int64_t)INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
   if constexpr (!f32 && OUT == OUT_V) {
-    if (a.G.n > 32 && !a.mask)
+    if (!a.mask && (a.G.n > 32 || (a.G.n >= 8 && !a.list && few_matrices(a.G, 1))))
       return launch_big(BIG_FUSED, a.G, a.rA, a.iA, a.rV, a.iV, a.rE, a.iE, a.info, a.itmax, a.flags, s, a.list,
                         a.list_count);
   }

@@ -161,7 +161,7 @@ __global__ __launch_bounds__(64) void k_eig(EigArgs a) {
   if (a.info && valid && g.r == 0) a.info[m] = nfail;
 }
 
-// Orders 33..64, eigenvalues only: the reduction by the whole workgroup on a
+// Orders 33..64 (and few matrices of a smaller order), eigenvalues only: the reduction by the whole workgroup on a
 // dense tile, then the iteration by its first wavefront in the same tile
 // (lahqr_stream; the others are done).  Order 48 x 16,384: 20.2 ms, against
 // 60.7 ms for one wavefront doing both on a 66 KB tile; at 41 KB four
@@ -194,8 +194,8 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_eig_block(E
   __syncthreads();  // the idle wavefronts keep their places (chain_wave) until the end
 }
 
-// Orders 33..64 that start from a Hessenberg matrix: one wavefront per matrix
-// on the banded tile
+// Orders 33..64 (and few matrices of a smaller order) that start from a
+// Hessenberg matrix: one wavefront per matrix on the banded tile
 template <int SRC>
 __global__ __launch_bounds__(64) void k_eig_band(EigArgs a) {
   extern __shared__ double2 lds[];
@@ -251,7 +251,8 @@ int launch_eig_block(const EigArgs &a, hipStream_t s) {
 template <int SRC, bool TZ>
 int launch_eig(const EigArgs &a, hipStream_t s) {
   if (a.G.nmat > (int64_t)INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
-  const int nb = nb_for(a.G.n);
+  int nb = nb_for(a.G.n);
+  if (!TZ && a.G.n >= 4 && few_matrices(a.G, SRC == SRC_MATRIX && a.G.n > 16 ? 1 : 4)) nb = 64;
   const int mpw = 64 / nb;
   const unsigned grid = (unsigned)((a.G.nmat + mpw - 1) / mpw);
   switch (nb) {
@@ -260,6 +261,8 @@ int launch_eig(const EigArgs &a, hipStream_t s) {
     case 32: hipLaunchKernelGGL((k_eig<32, 1, SRC, TZ>), dim3(grid), dim3(64), 0, s, a); break;
     default:
       if constexpr (SRC == SRC_MATRIX) {
+        if (a.G.n <= 16) return launch_eig_block<16, 4>(a, s);
+        if (a.G.n <= 32) return launch_eig_block<32, 4>(a, s);
         return a.G.n <= 48 ? launch_eig_block<48, 4>(a, s) : launch_eig_block<64, 4>(a, s);
       } else if constexpr (TZ) {
         return launch_big(BIG_ROOTS, a.G, a.rH, a.iH, a.rZ, a.iZ, a.rE, a.iE, a.info, a.itmax, 0, s, nullptr, nullptr,
