@@ -21,7 +21,8 @@
 //                  matrices of a wavefront then have (nearly) the same order.
 //                  Bins (16, 16) and (32, 32) run two such kernels instead,
 //                  k_reduce_var and k_qr_var (the banded path); the bins'
-//                  orders <= 12 and <= 24 in slots of capacity 12 and 24.
+//                  orders <= 12, and <= 24 and <= 28, in slots of capacity 12,
+//                  and 24 and 28.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -44,6 +45,14 @@ __host__ __device__ constexpr int var_p(int v) { return (v == 1 || v == 3) ? 2 :
 __host__ __device__ constexpr int default_variant(int n) { return n <= 8 ? 0 : (n <= 16 ? 2 : 4); }
 // orders of a width-16 / width-32 bin that run in slots of capacity 12 / 24
 __host__ __device__ constexpr int small_cut(int v) { return var_nb(v) == 16 ? 12 : (var_nb(v) == 32 ? 24 : 0); }
+// orders of a width-32 bin that run in slots of capacity 28 at most, as the
+// whole batches of one order do: a row of 28 spills 42 registers' worth where
+// one of 32 spills 114 (131,072 matrices of orders 4..32, with the scheduling
+// of k_qr_var: 21.3 -> 19.9 ms; the split alone 22.0, its parts being 4.4 turns
+// of the grid each)
+__host__ __device__ constexpr int mid_cut(int v) { return var_nb(v) == 32 ? 28 : var_nb(v); }
+
+constexpr int kParts = 3;  // of a bin, by capacity (bin_part)
 
 struct BinState {
   int32_t hist[kMaxN + 1];     // count per order
@@ -51,7 +60,9 @@ struct BinState {
   int64_t start[kBins];        // bin range in the permutation
   int64_t count[kBins];
   int64_t small[kBins];        // leading part of a bin with orders <= small_cut
+  int64_t mid[kBins];          // and with orders <= mid_cut
   int32_t var_of_n[kMaxN + 1]; // kernel variant per order
+  int32_t next[kBins][kParts]; // k_qr_var: sets of matrices taken past the grid's first
 };
 
 struct VarArgs {
@@ -80,6 +91,8 @@ __global__ void k_bin_init(BinState *b, const int8_t *var_table) {
     b->start[i] = 0;
     b->count[i] = 0;
     b->small[i] = 0;
+    b->mid[i] = 0;
+    for (int p = 0; p < kParts; ++p) b->next[i][p] = 0;
   }
 }
 
@@ -110,16 +123,31 @@ __global__ void k_bin_scan(BinState *b) {
       b->cursor[n] = (int32_t)pos;
       pos += b->hist[n];
       if (n <= small_cut(bi)) b->small[bi] = pos - b->start[bi];
+      if (n <= mid_cut(bi)) b->mid[bi] = pos - b->start[bi];
     }
     b->count[bi] = pos - b->start[bi];
   }
 }
 
+// A chunk of matrices per workgroup and turn: each takes its rank among the
+// chunk's matrices of its order from LDS, and one global atomic per order
+// present reserves their places (131,072 matrices of 29 orders: 248 us with an
+// atomic per matrix -> 9 us).
 __global__ void k_bin_scatter(VarArgs a) {
-  for (int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; m < a.nmat;
-       m += (int64_t)gridDim.x * blockDim.x) {
-    const int n = a.dims[m];
-    if (n >= 1 && n <= kMaxN) a.perm[atomicAdd(&a.bins->cursor[n], 1)] = (int32_t)m;
+  __shared__ int32_t cnt[kMaxN + 1], base[kMaxN + 1];
+  for (int64_t c0 = (int64_t)blockIdx.x * blockDim.x; c0 < a.nmat; c0 += (int64_t)gridDim.x * blockDim.x) {
+    if (threadIdx.x <= kMaxN) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t m = c0 + threadIdx.x;
+    const int n = m < a.nmat ? a.dims[m] : 0;
+    const bool in = n >= 1 && n <= kMaxN;
+    const int32_t rank = in ? atomicAdd(&cnt[n], 1) : 0;
+    __syncthreads();
+    if (threadIdx.x <= kMaxN && cnt[threadIdx.x])
+      base[threadIdx.x] = atomicAdd(&a.bins->cursor[threadIdx.x], cnt[threadIdx.x]);
+    __syncthreads();
+    if (in) a.perm[base[n] + rank] = (int32_t)m;
+    __syncthreads();  // cnt and base are rewritten for the next chunk
   }
 }
 
@@ -176,17 +204,13 @@ __global__ __launch_bounds__(64) void k_zgeev_var(VarArgs a, int bin) {
 // banded tile -- the LDS of a wavefront drops from 18.6 to 11.8 KB (NB = 16)
 // and from 33.8 to 19.5 KB (NB = 32), one more resident wavefront per SIMD.
 // Both walk the bin's range like k_zgeev_var.
-// the range of a bin, or of its part 0 (orders <= small_cut) or part 1 (the rest)
+// the range of a bin's part 0 (orders <= small_cut), 1 (<= mid_cut) or 2 (the rest)
 __device__ __forceinline__ void bin_part(const VarArgs &a, int bin, int part, int64_t &start, int64_t &count) {
-  start = a.bins->start[bin];
-  count = a.bins->count[bin];
-  const int64_t small = a.bins->small[bin];
-  if (part == 0) {
-    count = small;
-  } else if (part == 1) {
-    start += small;
-    count -= small;
-  }
+  const int64_t small = a.bins->small[bin], mid = a.bins->mid[bin];
+  const int64_t from = part == 0 ? 0 : (part == 1 ? small : mid);
+  const int64_t to = part == 0 ? small : (part == 1 ? mid : a.bins->count[bin]);
+  start = a.bins->start[bin] + from;
+  count = to - from;
 }
 
 template <int LG, int MPW>
@@ -227,6 +251,10 @@ __global__ __launch_bounds__(64 * reduce_waves<NB>()) __attribute__((amdgpu_wave
   }
 }
 
+// The largest orders first, and each wavefront takes the next set of matrices
+// when it is done with one: a set takes about a millisecond and a bin is only a
+// few turns of the grid, so with a fixed share each (4.4 turns were 5) the
+// whole grid waited for the last, whose orders are the largest.
 template <int NB, int LW>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(qr_band_waves<NB>()))) void k_qr_var(VarArgs a,
                                                                                                        int bin,
@@ -237,10 +265,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(qr_band_wave
   int64_t start, count;
   bin_part(a, bin, part, start, count);
   const int64_t nwaves = (count + MPW - 1) / MPW;
-  for (int64_t w = blockIdx.x; w < nwaves; w += gridDim.x) {
+  for (int64_t w = blockIdx.x; w < nwaves;) {
     int lane = threadIdx.x;
     asm volatile("" : "+v"(lane));
-    const int64_t idx = w * MPW + lane / G::LG;
+    const int64_t idx = (nwaves - 1 - w) * MPW + lane / G::LG;
     const bool valid = idx < count;
     const int64_t m = valid ? a.perm[start + idx] : 0;
     const int n = valid ? a.dims[m] : 0;
@@ -255,11 +283,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(qr_band_wave
         band_qr_one<NB, LW>(g, Gm, base, vbase, nmax, a.itmax, a.rV, a.iV, a.rE, a.iE, nullptr, nullptr);
     if (a.info && valid && g.r == 0) a.info[m] = nfail;
     wave_sync();
+    int32_t t = 0;
+    if (threadIdx.x == 0) t = atomicAdd(&a.bins->next[bin][part], 1);
+    w = (int64_t)gridDim.x + __builtin_amdgcn_readfirstlane(t);
   }
 }
 
 constexpr size_t kAlign = 256;
 constexpr size_t align_up(size_t x) { return (x + kAlign - 1) / kAlign * kAlign; }
+
+static_assert(align_up(sizeof(BinState)) == 768, "workspaces keep their size");
 
 size_t varsize_ws_bytes(int64_t nmat) {
   return align_up(sizeof(BinState)) + align_up((size_t)nmat * sizeof(int32_t));
@@ -311,11 +344,13 @@ int enqueue_varsize(int64_t nmat, const int32_t *dims, const int64_t *a_off, con
         break;
       case 3: hipLaunchKernelGGL((k_zgeev_var<16, 2>), dim3(g), dim3(64), 0, s, a, 3); break;
       default:
-        // orders <= 24 of the bin in slots of 24, the rest in slots of 32
+        // orders <= 24 of the bin in slots of 24, up to 28 in slots of 28, the rest in slots of 32
         hipLaunchKernelGGL((k_reduce_var<24, 32>), dim3(g), dim3(64 * reduce_waves<24>()), 0, s, a, 4, 0);
         hipLaunchKernelGGL((k_qr_var<24, 32>), dim3(g), dim3(64), 0, s, a, 4, 0);
-        hipLaunchKernelGGL((k_reduce_var<32, 0>), dim3(g), dim3(64 * reduce_waves<32>()), 0, s, a, 4, 1);
-        hipLaunchKernelGGL((k_qr_var<32, 0>), dim3(g), dim3(64), 0, s, a, 4, 1);
+        hipLaunchKernelGGL((k_reduce_var<28, 32>), dim3(g), dim3(64 * reduce_waves<28>()), 0, s, a, 4, 1);
+        hipLaunchKernelGGL((k_qr_var<28, 32>), dim3(g), dim3(64), 0, s, a, 4, 1);
+        hipLaunchKernelGGL((k_reduce_var<32, 0>), dim3(g), dim3(64 * reduce_waves<32>()), 0, s, a, 4, 2);
+        hipLaunchKernelGGL((k_qr_var<32, 0>), dim3(g), dim3(64), 0, s, a, 4, 2);
         break;
     }
   }
