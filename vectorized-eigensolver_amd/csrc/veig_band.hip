@@ -4,7 +4,8 @@
 //
 //   k_gehrd_c<NB, LW>  the Hessenberg reduction alone (zgehrd, Toolbox.hpp:
 //                      1315-1469) on the dense tile, by one wavefront (NB = 16)
-//                      or two sharing each update (NB = 24..32), written in
+//                      or two sharing each update (NB = 12), above order 16 by
+//                      one matrix per workgroup (veig_big.hip), written in
 //                      zgehrd's compact form -- H on and above the
 //                      subdiagonal, the reflector vectors v(i+2:n) below it,
 //                      tau(i) -- to the V and E planes, which serve as its
@@ -97,7 +98,18 @@ int launch_banded(const FusedArgs &a, hipStream_t s) {
   // a list launch gets the whole batch's grid: the list's length is only
   // known on the device, and it never exceeds the batch
   const unsigned grid = (unsigned)((a.G.nmat + mpw - 1) / mpw);
-  hipLaunchKernelGGL((k_gehrd_c<NB, LW>), dim3(grid), dim3(64 * reduce_waves<NB>()), 0, s, a);
+  if constexpr (NB > 16) {
+    // one matrix per workgroup, its row in two or four chunks: the lane groups'
+    // two dense tiles left one and a half wavefronts per SIMD (whole calls of
+    // 20,000 matrices, lane groups -> workgroups: order 17 2.50 -> 2.36 ms, 24
+    // 4.11 -> 3.86, 28 5.44 -> 5.25, 32 7.34 -> 7.0; eight chunks: 32 7.4,
+    // two: 7.3; up to order 24 two are the best, four 3.93)
+    const int st = launch_big(BIG_REDUCE, a.G, a.rA, a.iA, a.rV, a.iV, a.rE, a.iE, nullptr, 0, 0, s, a.list,
+                              a.list_count);
+    if (st != VEIG_OK) return st;
+  } else {
+    hipLaunchKernelGGL((k_gehrd_c<NB, LW>), dim3(grid), dim3(64 * reduce_waves<NB>()), 0, s, a);
+  }
   hipLaunchKernelGGL((k_qr_band<NB, LW>), dim3(grid), dim3(64), 0, s, a);
   VEIG_HIP(hipGetLastError());
   return VEIG_OK;

@@ -35,12 +35,11 @@ constexpr int qr_band_waves() { return NB <= 16 ? 3 : 2; }
 // Wavefronts of a workgroup that share one reduction, and the LDS it needs
 // beside the dense tiles: one partial product per wavefront and lane.  At
 // NB = 16 one wavefront (gehrd_compact) measured faster than two sharing
-// the work (7.6 vs 6.2 ms for 2^20 matrices): the tiles already allow two
-// wavefronts per SIMD there, against one at NB = 32 and half at NB = 64.
-// Slots narrower than their lane group (NB = 12 on 16 lanes) take the
-// shared form too, whose loads and stores skip the lanes past the slot.
+// the work (7.6 vs 6.2 ms for 2^20 matrices).  Slots narrower than their lane
+// group (NB = 12 on 16 lanes) take the shared form, whose loads and stores skip
+// the lanes past the slot.
 template <int NB>
-constexpr int reduce_waves() { return NB == 64 ? 4 : (NB == 16 ? 1 : 2); }
+constexpr int reduce_waves() { return NB == 16 ? 1 : 2; }
 
 template <int NB, int LW = 0>
 struct ReduceTiles {

@@ -248,6 +248,7 @@ int launch_reduce(const BigArgs &a, hipStream_t s) {
 template <int MODE>
 int reduce_for(const BigArgs &a, hipStream_t s) {
   if (a.G.n <= 16) return launch_reduce<16, 4, MODE>(a, s);
+  if (a.G.n <= 24) return launch_reduce<24, 2, MODE>(a, s);
   if (a.G.n <= 32) return launch_reduce<32, 4, MODE>(a, s);
   if (a.G.n <= 48) return launch_reduce<48, 4, MODE>(a, s);
   if (a.G.n <= 64) return launch_reduce<64, 4, MODE>(a, s);
@@ -291,6 +292,7 @@ int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, doub
     case BIG_FUSED:
       VEIG_TRY(reduce_for<RD_FUSED>(a, s));
       return schur_for<SC_FUSED>(a, s);
+    case BIG_REDUCE: return reduce_for<RD_FUSED>(a, s);
     case BIG_GEHRD: return reduce_for<RD_GEHRD>(a, s);
     case BIG_HESS: return reduce_for<RD_HESS>(a, s);
     case BIG_UNGHR: return reduce_for<RD_UNGHR>(a, s);

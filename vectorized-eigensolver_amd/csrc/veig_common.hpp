@@ -398,8 +398,9 @@ int launch_zgeev64(const FusedArgs &a, hipStream_t s);
 // place: zgehrd (A -> compact form, tau in E), hessenberg (also Q in B),
 // zunghr (reflectors in A, tau in E -> Q in A), zlahqr (H in A -> T, Z in B
 // updated, E), ztrevc (T in A, B <- B X); polynomial roots with their Schur
-// form (coefficients in C -> T in A, Z in B, E).
-enum { BIG_FUSED = 0, BIG_GEHRD = 1, BIG_HESS = 2, BIG_UNGHR = 3, BIG_LAHQR = 4, BIG_TREVC = 5, BIG_ROOTS = 6 };
+// form (coefficients in C -> T in A, Z in B, E); the fused path's reduction
+// alone, for the banded kernels (A -> compact form in B, tau in E).
+enum { BIG_FUSED = 0, BIG_GEHRD = 1, BIG_HESS = 2, BIG_UNGHR = 3, BIG_LAHQR = 4, BIG_TREVC = 5, BIG_ROOTS = 6, BIG_REDUCE = 7 };
 int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, double *iB, double *rE, double *iE,
                int32_t *info, int itmax, uint32_t flags, hipStream_t s, const int32_t *list = nullptr,
                const int32_t *list_count = nullptr, const double *rC = nullptr, const double *iC = nullptr);

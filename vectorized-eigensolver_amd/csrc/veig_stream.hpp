@@ -1,5 +1,6 @@
-// One matrix per workgroup at orders 33..96: the pieces of the FP64 solve that
-// its kernels (veig_large.hip, veig_big.hip, veig_roots.hip) are made of.
+// One matrix per workgroup (orders 33..96, and lower ones in small batches): the pieces
+// of the FP64 solve that the kernels of veig_big.hip, veig_roots.hip and
+// veig_varsize.hip are made of.
 //
 //   reduce_block    the Hessenberg reduction on a dense LDS tile, every thread
 //                   owning a chunk of one row (right update) or column (left);

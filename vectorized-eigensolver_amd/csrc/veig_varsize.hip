@@ -20,7 +20,8 @@
 //                  range, read from device memory, wavefront by wavefront; the
 //                  matrices of a wavefront then have (nearly) the same order.
 //                  Bins (16, 16) and (32, 32) run two such kernels instead,
-//                  k_reduce_var and k_qr_var (the banded path); the bins'
+//                  k_reduce_var (above order 16 k_reduce_block_var) and
+//                  k_qr_var (the banded path); the bins'
 //                  orders <= 12, and <= 24 and <= 28, in slots of capacity 12,
 //                  and 24 and 28.
 #include <hip/hip_runtime.h>
@@ -31,6 +32,7 @@
 #include <vector>
 
 #include "veig_band.hpp"
+#include "veig_stream.hpp"
 
 using namespace veig;
 
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(64) void k_zgeev_var(VarArgs a, int bin) {
 }
 
 // Bins (16, 16) and (32, 32) on the two-kernel banded path (one index per
-// lane): k_reduce_var<NB> writes each matrix's compact Hessenberg form into
+// lane): k_reduce_var<NB> (k_reduce_block_var above order 16) writes each matrix's compact Hessenberg form into
 // its V and E slots, then k_qr_var<NB> forms Q, iterates and solves on the
 // banded tile -- the LDS of a wavefront drops from 18.6 to 11.8 KB (NB = 16)
 // and from 33.8 to 19.5 KB (NB = 32), one more resident wavefront per SIMD.
@@ -248,6 +250,34 @@ __global__ __launch_bounds__(64 * reduce_waves<NB>()) __attribute__((amdgpu_wave
     Gm.n = n;
     const int64_t base = valid ? a.a_off[m] : 0, vbase = valid ? a.e_off[m] : 0;
     band_reduce_one<NB, LW>(sm, n, Gm, base, vbase, nmax, a.rA, a.iA, a.rV, a.iV, a.rE, a.iE);
+  }
+}
+
+// The reduction of a width-32 bin's part, one matrix per workgroup at a time, as
+// the whole batches' is above order 16 (131,072 matrices of orders 4..32: the
+// bin's reductions 3.15 -> 2.5 ms, the call 19.9 -> 19.2 ms)
+template <int CAP, int W>
+__global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce_block_var(VarArgs a, int bin, int part) {
+  __shared__ ReduceBlock<CAP, W> sm;
+  __shared__ double2 tau[CAP];
+  int64_t start, count;
+  bin_part(a, bin, part, start, count);
+  for (int64_t w = blockIdx.x; w < count; w += gridDim.x) {
+    const int64_t m = a.perm[start + w];
+    const int n = a.dims[m];
+    Geom Gm;
+    Gm.nmat = 0;
+    Gm.T = 1;
+    Gm.n = n;
+    reduce_load(sm, n, Gm, a.a_off[m], a.rA, a.iA);
+    reduce_block(sm, n, tau);
+    reduce_store(sm, n, Gm, a.a_off[m], a.rV, a.iV);
+    if ((int)threadIdx.x + 1 < n) {
+      const cx<double> t = ld<double>(tau + threadIdx.x);
+      a.rE[a.e_off[m] + threadIdx.x] = t.re;
+      a.iE[a.e_off[m] + threadIdx.x] = t.im;
+    }
+    __syncthreads();  // the tile and tau are rewritten for the next matrix
   }
 }
 
@@ -345,11 +375,11 @@ int enqueue_varsize(int64_t nmat, const int32_t *dims, const int64_t *a_off, con
       case 3: hipLaunchKernelGGL((k_zgeev_var<16, 2>), dim3(g), dim3(64), 0, s, a, 3); break;
       default:
         // orders <= 24 of the bin in slots of 24, up to 28 in slots of 28, the rest in slots of 32
-        hipLaunchKernelGGL((k_reduce_var<24, 32>), dim3(g), dim3(64 * reduce_waves<24>()), 0, s, a, 4, 0);
+        hipLaunchKernelGGL((k_reduce_block_var<24, 2>), dim3(2 * g), dim3(ReduceBlock<24, 2>::kThreads), 0, s, a, 4, 0);
         hipLaunchKernelGGL((k_qr_var<24, 32>), dim3(g), dim3(64), 0, s, a, 4, 0);
-        hipLaunchKernelGGL((k_reduce_var<28, 32>), dim3(g), dim3(64 * reduce_waves<28>()), 0, s, a, 4, 1);
+        hipLaunchKernelGGL((k_reduce_block_var<32, 4>), dim3(2 * g), dim3(ReduceBlock<32, 4>::kThreads), 0, s, a, 4, 1);
         hipLaunchKernelGGL((k_qr_var<28, 32>), dim3(g), dim3(64), 0, s, a, 4, 1);
-        hipLaunchKernelGGL((k_reduce_var<32, 0>), dim3(g), dim3(64 * reduce_waves<32>()), 0, s, a, 4, 2);
+        hipLaunchKernelGGL((k_reduce_block_var<32, 4>), dim3(2 * g), dim3(ReduceBlock<32, 4>::kThreads), 0, s, a, 4, 2);
         hipLaunchKernelGGL((k_qr_var<32, 0>), dim3(g), dim3(64), 0, s, a, 4, 2);
         break;
     }
