@@ -96,3 +96,25 @@ def test_stages_either_side(gpu, n, N):
     veig.ztrevc(n, N // 6, 6, rH, iH, rZ, iZ)
     V = back(rZ, iZ)
     assert np.all(H.backward_error(A, E, V) <= 64 * n * np.finfo(float).eps)
+
+
+@pytest.mark.parametrize("n", [65, 66, 79, 80])
+def test_orders_above_64_past_two_matrices_per_cu(gpu, n):
+    # few: four segments of 20 columns per Schur vector; many: two of 40
+    A = H.gaussian(4, n, 8500 + n)
+    big = np.tile(A, (129, 1, 1))  # 516
+    Eo, Vo, _ = H.oracle_eig(A, 1)
+    E, V, info = gpu_eig(big, 4)
+    assert np.all(info == 0)
+    check_parity(A, E[:4], V[:4], info[:4], Eo, Vo)
+    check_parity(A, E[-4:], V[-4:], info[-4:], Eo, Vo)
+    N = len(big)
+    rH, iH = planes(big, 4)
+    rZ, iZ = torch.empty_like(rH), torch.empty_like(iH)
+    rE, iE = (torch.empty(N * n, dtype=torch.float64, device="cuda") for _ in range(2))
+    veig.hessenberg(n, N // 4, 4, rH, iH, rZ, iZ)
+    veig.zlahqr(n, N // 4, 4, rE, iE, rH, iH, rZ, iZ)
+    Es = values(rE, iE, n, 4)
+    veig.ztrevc(n, N // 4, 4, rH, iH, rZ, iZ)
+    Vs = H.from_soa(rZ.cpu().numpy(), iZ.cpu().numpy(), n, 4)
+    assert np.all(H.backward_error(big, Es, Vs) <= 64 * n * np.finfo(float).eps)

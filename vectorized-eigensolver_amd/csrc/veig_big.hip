@@ -14,18 +14,18 @@
 //                      sweeps (SchurRows); then the eigenvector solve and
 //                      V = Z X on the matrix cores.
 //
-// Segments: the row of a Schur vector is cut so that a lane's part fits the
-// registers of three wavefronts per SIMD: two segments of 24 or 32 columns up
-// to order 64, four of 20 or 24 above (wider rows, the same registers).  LDS
-// is allocated for the batch's order: 40 KB at n = 64 (four matrices per CU),
-// 76 KB at n = 88 (two).  Up to 24 columns the allocation is held to four
-// wavefronts per SIMD although that spills (order 48 x 8,192: 12.3 -> 11.5 ms,
-// order 79 x 3,328: 51 -> 34 ms, whose two workgroups of six wavefronts do not
-// share a CU at three), at 32 columns to three.
+// Segments: the row of a Schur vector is cut in two, of 16 to 32 columns up to
+// order 64 (three or four wavefronts per SIMD), of 40 or 48 above (two, which
+// the LDS of 60 to 90 KB per workgroup leaves in any case): half the wavefronts,
+// and less ring, than four segments of 20 or 24 (3,328 matrices: order 65 24.4
+// -> 22.4 ms, 79 34.4 -> 31.6, 88 45.7 -> 39.0).  Up to 24 columns the allocation
+// is held to four wavefronts per SIMD although that spills (order 48 x 8,192:
+// 12.3 -> 11.5 ms), at 32 columns to three.  LDS is allocated for the batch's
+// order: 40 KB at n = 64 (four matrices per CU), 71 KB at n = 88 (two).
 //
 // Measured, whole passes (in brackets the kernels these replaced, whose bulge
 // chase went through LDS): order 64 x 65,536 181 ms (371), order 79 x 3,328
-// 36 ms (233: a workgroup barrier per half step and Z in global memory), the
+// 34 ms (233: a workgroup barrier per half step and Z in global memory), the
 // stages hessenberg + zlahqr + ztrevc at order 40 x 2,048 3.1 ms (21).  What
 // bounds order 64 is instruction issue, the chain wavefront's (7,700 steps of
 // about 88 instructions and 230 sweeps of about 480 more per matrix) and,
@@ -123,7 +123,7 @@ constexpr int schur_threads() {
 
 // wavefronts per SIMD the register allocation is held to
 template <int SL>
-constexpr int schur_waves() { return SL <= 24 ? 4 : 3; }
+constexpr int schur_waves() { return SL <= 24 ? 4 : (SL <= 32 ? 3 : 2); }
 
 template <int SL, int NT, int MODE>
 __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_waves_per_eu(schur_waves<SL>()))) void k_schur(BigArgs a) {
@@ -274,8 +274,11 @@ int schur_for(const BigArgs &a, hipStream_t s) {
   if (a.G.n <= 40) return launch_schur<20, 2, MODE>(a, s);
   if (a.G.n <= 48) return launch_schur<24, 2, MODE>(a, s);
   if (a.G.n <= 64) return launch_schur<32, 2, MODE>(a, s);
-  if (a.G.n <= 80) return launch_schur<20, 4, MODE>(a, s);
-  return launch_schur<24, 4, MODE>(a, s);
+  // two matrices per CU at most: the shorter segments replay sooner (order 79 x
+  // 64: 3.96 against 4.11 ms), past that the fewer wavefronts win
+  if (a.G.n <= 80 && few_matrices(a.G, 2)) return launch_schur<20, 4, MODE>(a, s);
+  if (a.G.n <= 80) return launch_schur<40, 2, MODE>(a, s);
+  return launch_schur<48, 2, MODE>(a, s);
 }
 
 }  // namespace

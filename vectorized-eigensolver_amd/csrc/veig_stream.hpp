@@ -808,14 +808,15 @@ struct SchurRows {
         if (dn) rot_right(qd, zd, z[0]);
       }
       // ---- steps 0..SL-2 of each segment, kStep at a time where any is live ----
-      unsigned kmask = 0;
+      using Mask = std::conditional_t<(SL > 32), uint64_t, unsigned>;
+      Mask kmask = 0;
 #pragma unroll
       for (int g = 0; g < NT; ++g) {
         const int sg = cur - g < 0 ? cur - g + R : cur - g;
         const int lo = __builtin_amdgcn_readfirstlane(ring.L[sg]) - SL * g;
         const int hi = __builtin_amdgcn_readfirstlane(ring.I[sg]) - SL * g;
         const int l = lo < 0 ? 0 : (lo > SL - 1 ? SL - 1 : lo), e = hi < 0 ? 0 : (hi > SL - 1 ? SL - 1 : hi);
-        kmask |= e > l ? ((1u << e) - 1u) & ~((1u << l) - 1u) : 0u;
+        kmask |= e > l ? ((Mask(1) << e) - 1u) & ~((Mask(1) << l) - 1u) : Mask(0);
       }
       static_for<(SL + kStep - 1) / kStep>([&](auto bc) {
         constexpr int b = decltype(bc)::value * kStep;
