@@ -1,0 +1,78 @@
+"""Infinities and NaN where an operation does not read them: what the reduction
+has finished, what an eigenvector or a deflated block does not depend on.  The
+rest of the result is finite and holds the properties that it has without them
+(tolerances as in test_gpu_routes)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import helpers as H
+import veig
+
+pytestmark = pytest.mark.gpu
+BAD = [np.inf, np.nan]
+
+
+def planes(A):
+    return tuple(torch.from_numpy(x).cuda() for x in H.to_soa(A, 1))
+
+
+def zeros(count):
+    return tuple(torch.zeros(count, dtype=torch.float64, device="cuda") for _ in range(2))
+
+
+def back(p, n):
+    return H.from_soa(p[0].cpu().numpy(), p[1].cpu().numpy(), n, 1)
+
+
+def vec(p, n):
+    return H.vec_from_soa(p[0].cpu().numpy(), p[1].cpu().numpy(), n, 1)
+
+
+def norm(X):
+    return np.linalg.norm(X, axis=(-2, -1))
+
+
+# (order, matrices): one matrix per workgroup in every capacity, and the lane
+# groups of the orders up to 16
+SIZES = [(8, 3), (16, 3), (17, 3), (24, 3), (32, 3), (33, 3), (48, 3), (64, 3), (80, 3), (96, 3), (16, 1027)]
+
+
+@pytest.mark.parametrize("bad", BAD)
+@pytest.mark.parametrize("n,N", SIZES)
+def test_reduction_first_row(gpu, n, N, bad):
+    # no reflector and no update from the left reads row 0, and no update from
+    # the right mixes it with others: Q and the rows below are those of the
+    # matrix with any other first row
+    A = np.tile(H.gaussian(1, n, 9000 + n), (N, 1, 1))
+    for m, c in enumerate((0, n // 2, n - 1)):
+        A[m, 0, c] = bad
+    a, q = planes(A), zeros(A.size)
+    veig.hessenberg(n, N, 1, *a, *q)
+    b, t = planes(A), zeros(N * n)
+    veig.zgehrd(n, N, 1, *b, *t)
+    Hs, Q, tol = np.triu(back(a, n), -1), back(q, n), 1e-13 * n
+    assert np.all(norm(Q @ np.conj(np.swapaxes(Q, 1, 2)) - np.eye(n)) <= tol)
+    assert np.all(Q[:, 0, 1:] == 0) and np.all(Q[:, 1:, 0] == 0)
+    R = A[:, 1:] @ Q - Q[:, 1:, 1:] @ Hs[:, 1:]
+    assert np.all(norm(R) <= tol * norm(A[:, 1:]))
+    assert np.array_equal(back(b, n)[:, 1:], back(a, n)[:, 1:])
+    assert np.all(np.isfinite(vec(t, n)))
+
+
+@pytest.mark.parametrize("n", [17, 24, 32, 33, 48, 64, 80, 96])
+def test_q_columns_before_a_reflector(gpu, n):
+    # reflector i changes columns i+1..n-1 of Q only
+    a, t = planes(H.gaussian(1, n, 9100 + n)), zeros(n)
+    veig.zgehrd(n, 1, 1, *a, *t)
+    C = back(a, n)
+    ref = planes(C)
+    veig.zunghr(n, 1, 1, *ref, *t)
+    for i in (0, 1, n // 2, n - 3):
+        B = C.copy()
+        B[0, n - 1, i] = np.nan
+        q = planes(B)
+        veig.zunghr(n, 1, 1, *q, *t)
+        assert np.all(np.abs(back(ref, n) - back(q, n))[:, :, :i + 1] <= 1e-13 * n)

@@ -80,12 +80,17 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce(BigA
   if (!block_matrix(a, m)) return;  // workgroup-uniform
   const int n = a.G.n, tid = threadIdx.x, r = tid % CAP, q = tid / CAP;
   const int64_t base = a.G.mat_base(m), vb = a.G.vec_base(m);
-  reduce_load(sm, n, a.G, base, a.rA, a.iA);
+  unsigned top = 0;
   if constexpr (MODE == RD_UNGHR) {
-    if (tid + 1 < n) st<double>(tau + tid, mk<double>(a.rE[vb + a.G.ve(tid)], a.iE[vb + a.G.ve(tid)]));
-    __syncthreads();
+    if (tid + 1 < n) {
+      const cx<double> t = mk<double>(a.rE[vb + a.G.ve(tid)], a.iE[vb + a.G.ve(tid)]);
+      top = high_word(t);
+      st<double>(tau + tid, t);
+    }
+    top = reduce_load(sm, n, a.G, base, a.rA, a.iA, top);
   } else {
-    reduce_block(sm, n, tau);
+    top = reduce_load(sm, n, a.G, base, a.rA, a.iA);
+    reduce_block(sm, n, top, tau);
     const bool fused = MODE == RD_FUSED;
     reduce_store(sm, n, a.G, base, fused ? a.rB : a.rA, fused ? a.iB : a.iA);
     if (a.rE && tid + 1 < n) {
@@ -95,9 +100,13 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce(BigA
     }
   }
   if constexpr (MODE == RD_HESS || MODE == RD_UNGHR) {
+    double *re = MODE == RD_HESS ? a.rB : a.rA, *im = MODE == RD_HESS ? a.iB : a.iA;
+    if (__builtin_expect(top >= kNonFinite, 0)) {
+      form_q_rare(sm, n, tau, a.G, base, re, im);
+      return;
+    }
     cx<double> z[S::CH];
     form_q_block(sm, n, tau, z);
-    double *re = MODE == RD_HESS ? a.rB : a.rA, *im = MODE == RD_HESS ? a.iB : a.iA;
 #pragma unroll
     for (int j = 0; j < S::CH; ++j) {
       const int c = q * S::CH + j;

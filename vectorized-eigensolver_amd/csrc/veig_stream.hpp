@@ -89,6 +89,26 @@ __device__ __forceinline__ double wave_sum(double x) {
   return (read_lane(x, 0) + read_lane(x, 16)) + (read_lane(x, 32) + read_lane(x, 48));
 }
 
+// the bits above the low word, without the sign: ordered as the magnitudes are,
+// an infinity or a NaN from kNonFinite on
+constexpr unsigned kNonFinite = 0x7ff00000u;
+__device__ __forceinline__ unsigned high_word(double x) {
+  return (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32) & 0x7fffffffu;
+}
+__device__ __forceinline__ unsigned high_word(cx<double> x) { return max(high_word(x.re), high_word(x.im)); }
+
+// the largest over the workgroup, in every thread (one barrier; words: one LDS
+// word per wavefront)
+__device__ __forceinline__ unsigned block_max(unsigned x, unsigned *words) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x = max(x, (unsigned)__shfl_xor((int)x, o));
+  if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = x;
+  __syncthreads();
+  unsigned m = 0;
+  for (int w = 0; w < (int)(blockDim.x >> 6); ++w) m = max(m, words[w]);
+  return (unsigned)__builtin_amdgcn_readfirstlane((int)m);
+}
+
 // --------------------------------------------------------------------------
 // The Hessenberg reduction (zgehrd, Toolbox.hpp:1315-1469, with zlarfg's
 // LAPACK sign and its x = 0 guard) of the n x n matrix in a dense tile of
@@ -100,21 +120,28 @@ __device__ __forceinline__ double wave_sum(double x) {
 // wavefront forms the reflector from column i (the same arithmetic on the same
 // data).  Five barriers per reflector.  The tile is zero outside the matrix,
 // so chunks need no bounds inside.
+// kRare (the input holds an infinity or a NaN): a chunk's entries before the
+// reflector's first are left out, not multiplied by the zeros of v, which would
+// carry on what a finished row or column holds.  Entry by entry from LDS, and
+// apart from the usual input's code: masks there cost order 64 x 65,536 180.4 ->
+// 183.4 ms, the stages at order 40 x 2,048 3.09 -> 3.30.
 // --------------------------------------------------------------------------
 template <int CAP, int W>
 struct ReduceBlock {
   static constexpr int LD = CAP | 1;  // odd: row-wise walks start on distinct banks
   static constexpr int CH = CAP / W;
   static constexpr int kThreads = (CAP * W + 63) / 64 * 64;
+  static_assert(kThreads / 64 <= 12, "a word per wavefront");
   static_assert(LD == CAP + 1, "the reflector lives in the padding row");
   double2 H[LD * CAP];
   double2 part[W * CAP];
+  unsigned words[12];  // block_max
   __device__ __forceinline__ double2 *at(int r, int c) { return H + c * LD + r; }
   __device__ __forceinline__ double2 *v(int c) { return H + c * LD + CAP; }  // the reflector's entry c
 };
 
-template <int CAP, int W>
-__device__ __forceinline__ void reduce_block(ReduceBlock<CAP, W> &sm, int n, double2 *tau_out) {
+template <bool kRare, int CAP, int W>
+__device__ __forceinline__ void reduce_steps(ReduceBlock<CAP, W> &sm, int n, double2 *tau_out) {
   using R = double;
   constexpr int CH = ReduceBlock<CAP, W>::CH;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -145,17 +172,23 @@ __device__ __forceinline__ void reduce_block(ReduceBlock<CAP, W> &sm, int n, dou
     if (tau_out && tid == 0) st<R>(tau_out + i, tau);
     __syncthreads();
     const bool mine = in && c0 + CH - 1 > i && c0 < n;
+    const int cr = c0 > i ? c0 : i + 1, ce = min(c0 + CH, n);  // kRare: these of the chunk
     // ---- H <- H (I - tau v v^H): row r, columns of the chunk ----
     cx<R> h[CH], v[CH];
     cx<R> w = mk<R>(0, 0);
     if (mine) {
+      if constexpr (kRare) {
+#pragma unroll 1
+        for (int c = cr; c < ce; ++c) w = add(w, mul(ld<R>(sm.at(r, c)), ld<R>(sm.v(c))));
+      } else {
 #pragma unroll
-      for (int j = 0; j < CH; ++j) {
-        h[j] = ld<R>(sm.at(r, c0 + j));
-        v[j] = ld<R>(sm.v(c0 + j));  // zero at c <= i and beyond n
+        for (int j = 0; j < CH; ++j) {
+          h[j] = ld<R>(sm.at(r, c0 + j));
+          v[j] = ld<R>(sm.v(c0 + j));  // zero at c <= i and beyond n
+        }
+#pragma unroll
+        for (int j = 0; j < CH; ++j) w = add(w, mul(h[j], v[j]));
       }
-#pragma unroll
-      for (int j = 0; j < CH; ++j) w = add(w, mul(h[j], v[j]));
     }
     if (q < W) st<R>(sm.part + q * CAP + r, w);
     __syncthreads();
@@ -165,19 +198,29 @@ __device__ __forceinline__ void reduce_block(ReduceBlock<CAP, W> &sm, int n, dou
 #pragma unroll
       for (int p = 0; p < W; ++p) w = add(w, ld<R>(sm.part + p * CAP + r));
       w = mul(tau, w);
+      if constexpr (kRare) {
+#pragma unroll 1
+        for (int c = cr; c < ce; ++c) st<R>(sm.at(r, c), sub(ld<R>(sm.at(r, c)), mulc(w, ld<R>(sm.v(c)))));
+      } else {
 #pragma unroll
-      for (int j = 0; j < CH; ++j)
-        if (c0 + j > i) st<R>(sm.at(r, c0 + j), sub(h[j], mulc(w, v[j])));
+        for (int j = 0; j < CH; ++j)
+          if (c0 + j > i) st<R>(sm.at(r, c0 + j), sub(h[j], mulc(w, v[j])));
+      }
     }
     __syncthreads();
     // ---- H <- (I - conj(tau) v v^H) H: column r > i, rows of the chunk ----
     const bool left = mine && r > i;
     cx<R> y = mk<R>(0, 0);
     if (left) {
+      if constexpr (kRare) {
+#pragma unroll 1
+        for (int c = cr; c < ce; ++c) y = add(y, cmul(ld<R>(sm.v(c)), ld<R>(sm.at(c, r))));
+      } else {
 #pragma unroll
-      for (int j = 0; j < CH; ++j) h[j] = ld<R>(sm.at(c0 + j, r));
+        for (int j = 0; j < CH; ++j) h[j] = ld<R>(sm.at(c0 + j, r));
 #pragma unroll
-      for (int j = 0; j < CH; ++j) y = add(y, cmul(v[j], h[j]));
+        for (int j = 0; j < CH; ++j) y = add(y, cmul(v[j], h[j]));
+      }
     }
     if (q < W) st<R>(sm.part + q * CAP + r, y);
     __syncthreads();
@@ -186,20 +229,41 @@ __device__ __forceinline__ void reduce_block(ReduceBlock<CAP, W> &sm, int n, dou
 #pragma unroll
       for (int p = 0; p < W; ++p) y = add(y, ld<R>(sm.part + p * CAP + r));
       y = cmul(tau, y);  // conj(tau) * y
+      if constexpr (kRare) {
+#pragma unroll 1
+        for (int c = cr; c < ce; ++c) st<R>(sm.at(c, r), sub(ld<R>(sm.at(c, r)), mul(ld<R>(sm.v(c)), y)));
+      } else {
 #pragma unroll
-      for (int j = 0; j < CH; ++j)
-        if (c0 + j > i) st<R>(sm.at(c0 + j, r), sub(h[j], mul(v[j], y)));
+        for (int j = 0; j < CH; ++j)
+          if (c0 + j > i) st<R>(sm.at(c0 + j, r), sub(h[j], mul(v[j], y)));
+      }
     }
     __syncthreads();
   }
 }
 
-// the tile from memory, zeros outside the matrix (ends at a barrier)
+// (a call: inlined, it cost the usual input's kernels 1 to 3%, in registers and
+// in the order that the rest came out in)
 template <int CAP, int W>
-__device__ __forceinline__ void reduce_load(ReduceBlock<CAP, W> &sm, int n, const Geom &G, int64_t base,
-                                            const double *re, const double *im) {
+__device__ __noinline__ void reduce_rare(ReduceBlock<CAP, W> *sm, int n, double2 *tau_out) {
+  reduce_steps<true>(*sm, n, tau_out);
+}
+
+// top: the largest high word of the input, from reduce_load
+template <int CAP, int W>
+__device__ __forceinline__ void reduce_block(ReduceBlock<CAP, W> &sm, int n, unsigned top, double2 *tau_out) {
+  if (__builtin_expect(top >= kNonFinite, 0)) reduce_rare(&sm, n, tau_out);
+  else reduce_steps<false>(sm, n, tau_out);
+}
+
+// the tile from memory, zeros outside the matrix (ends at a barrier); returns
+// the largest high word of the matrix and of the thread's `also`
+template <int CAP, int W>
+__device__ __forceinline__ unsigned reduce_load(ReduceBlock<CAP, W> &sm, int n, const Geom &G, int64_t base,
+                                                const double *re, const double *im, unsigned also = 0) {
   constexpr int CH = ReduceBlock<CAP, W>::CH;
   const int r = threadIdx.x % CAP, q = threadIdx.x / CAP;
+  unsigned top = also;
   if (q < W) {
     cx<double> x[CH];
 #pragma unroll
@@ -212,9 +276,12 @@ __device__ __forceinline__ void reduce_load(ReduceBlock<CAP, W> &sm, int n, cons
       }
     }
 #pragma unroll
-    for (int j = 0; j < CH; ++j) st<double>(sm.at(r, q * CH + j), x[j]);
+    for (int j = 0; j < CH; ++j) {
+      top = max(top, high_word(x[j]));
+      st<double>(sm.at(r, q * CH + j), x[j]);
+    }
   }
-  __syncthreads();
+  return block_max(top, sm.words);
 }
 
 // the tile to memory
@@ -236,9 +303,8 @@ __device__ __forceinline__ void reduce_store(ReduceBlock<CAP, W> &sm, int n, con
 }
 
 // Q = H_0 H_1 ... H_{n-2} (zunghr, Toolbox.hpp:1470-1659) from the compact
-// form in the tile, thread (r, q) holding its chunk of row r in registers;
-// one barrier per reflector (the partial sums alternate between two halves of
-// the scratch, part and the vector's and tau's neighbours being free)
+// form in the tile, thread (r, q) holding its chunk of row r in registers; two
+// barriers per reflector, before and after the partial sums are read
 template <int CAP, int W>
 __device__ __forceinline__ void form_q_block(ReduceBlock<CAP, W> &sm, int n, const double2 *tau_in,
                                              cx<double> (&z)[ReduceBlock<CAP, W>::CH]) {
@@ -272,6 +338,40 @@ __device__ __forceinline__ void form_q_block(ReduceBlock<CAP, W> &sm, int n, con
 #pragma unroll
       for (int j = 0; j < CH; ++j) z[j] = sub(z[j], mulc(w, v[j]));
     }
+    __syncthreads();
+  }
+}
+
+// form_q_block for an input that holds an infinity or a NaN (see reduce_block):
+// a reflector leaves the columns before its first alone.  The chunk is kept in
+// the output planes, each thread using its own entries only.
+template <int CAP, int W>
+__device__ __forceinline__ void form_q_rare(ReduceBlock<CAP, W> &sm, int n, const double2 *tau_in, const Geom &G,
+                                            int64_t base, double *re, double *im) {
+  using R = double;
+  constexpr int CH = ReduceBlock<CAP, W>::CH;
+  const int r = threadIdx.x % CAP, q = threadIdx.x / CAP, c0 = q * CH;
+  const int end = q < W && r < n ? min(c0 + CH, n) : 0;
+  auto get = [&](int c) { return mk<R>(re[base + G.el(r, c)], im[base + G.el(r, c)]); };
+  auto put = [&](int c, cx<R> x) {
+    re[base + G.el(r, c)] = x.re;
+    im[base + G.el(r, c)] = x.im;
+  };
+  for (int c = c0; c < end; ++c) put(c, mk<R>(c == r ? 1.0 : 0.0, 0.0));
+  for (int i = 0; i + 1 < n; ++i) {
+    const int cr = c0 > i ? c0 : i + 1;
+    auto v = [&](int c) { return c == i + 1 ? mk<R>(1, 0) : ld<R>(sm.at(c, i)); };
+    cx<R> w = mk<R>(0, 0);
+#pragma unroll 1
+    for (int c = cr; c < end; ++c) w = add(w, mul(get(c), v(c)));
+    if (q < W) st<R>(sm.part + q * CAP + r, w);
+    __syncthreads();
+    w = mk<R>(0, 0);
+    if (q < W)
+      for (int p = 0; p < W; ++p) w = add(w, ld<R>(sm.part + p * CAP + r));
+    w = mul(ld<R>(tau_in + i), w);
+#pragma unroll 1
+    for (int c = cr; c < end; ++c) put(c, sub(get(c), mulc(w, v(c))));
     __syncthreads();
   }
 }

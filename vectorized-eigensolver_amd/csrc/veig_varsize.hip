@@ -256,8 +256,11 @@ __global__ __launch_bounds__(64 * reduce_waves<NB>()) __attribute__((amdgpu_wave
 // The reduction of a width-32 bin's part, one matrix per workgroup at a time, as
 // the whole batches' is above order 16 (131,072 matrices of orders 4..32: the
 // bin's reductions 3.15 -> 2.5 ms, the call 19.9 -> 19.2 ms)
+// (four wavefronts per SIMD at order 32, as its registers allow: 140 instead of
+// 128, three wavefronts, took 19.8 ms against 19.5)
 template <int CAP, int W>
-__global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce_block_var(VarArgs a, int bin, int part) {
+__global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) __attribute__((amdgpu_waves_per_eu(CAP > 24 ? 4 : 2)))
+void k_reduce_block_var(VarArgs a, int bin, int part) {
   __shared__ ReduceBlock<CAP, W> sm;
   __shared__ double2 tau[CAP];
   int64_t start, count;
@@ -269,8 +272,8 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce_bloc
     Gm.nmat = 0;
     Gm.T = 1;
     Gm.n = n;
-    reduce_load(sm, n, Gm, a.a_off[m], a.rA, a.iA);
-    reduce_block(sm, n, tau);
+    const unsigned top = reduce_load(sm, n, Gm, a.a_off[m], a.rA, a.iA);
+    reduce_block(sm, n, top, tau);
     reduce_store(sm, n, Gm, a.a_off[m], a.rV, a.iV);
     if ((int)threadIdx.x + 1 < n) {
       const cx<double> t = ld<double>(tau + threadIdx.x);
