@@ -76,3 +76,28 @@ def test_q_columns_before_a_reflector(gpu, n):
         q = planes(B)
         veig.zunghr(n, 1, 1, *q, *t)
         assert np.all(np.abs(back(ref, n) - back(q, n))[:, :, :i + 1] <= 1e-13 * n)
+
+
+@pytest.mark.parametrize("bad", BAD)
+@pytest.mark.parametrize("n", [16, 17, 24, 31, 32, 33, 48, 64, 65, 80, 96])
+def test_eigenvectors_that_do_not_depend_on_it(gpu, n, bad):
+    # eigenvector k depends on T(i, j) for i <= j <= k, row r of its result on R(r, j) for j <= k
+    T = np.triu(H.gaussian(1, n, 9200 + n))[0] + np.diag(3.0 * np.arange(n))
+    R = np.linalg.qr(H.gaussian(1, n, 9300 + n)[0])[0]
+    ref = planes(R[None])
+    veig.ztrevc(n, 1, 1, *planes(T[None]), *ref)
+    ref, tol = back(ref, n)[0], 1e-13 * n
+    for i, j in ((0, n // 2), (n // 2 - 1, n - 1), (n // 2, n // 2), (0, 1)):
+        B = T.copy()
+        B[i, j] = bad
+        v = planes(R[None])
+        veig.ztrevc(n, 1, 1, *planes(B[None]), *v)
+        assert np.all(np.abs(back(v, n)[0] - ref)[:, :j] <= tol * np.abs(ref).max())
+    for r, j in ((0, n - 1), (n - 1, n // 2), (n // 2, 1)):
+        Z = R.copy()
+        Z[r, j] = bad
+        v = planes(Z[None])
+        veig.ztrevc(n, 1, 1, *planes(T[None]), *v)
+        diff = np.abs(back(v, n)[0] - ref)
+        assert np.all(diff[r, :j] <= tol * np.abs(ref).max())
+        assert np.all(np.delete(diff, r, axis=0) <= tol * np.abs(ref).max())

@@ -176,6 +176,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
   const int zi = w < hw ? w : w - 1;
   if (w == hw) {
     // ---------------- the iteration and the eigenvector solve ----------------
+    const unsigned top = wave_top(t.h, BandTile::entries(n), lane);
     __builtin_amdgcn_s_setprio(3);  // the workgroup waits for the chain: it issues first on its SIMD
     if constexpr (MODE != SC_TREVC) {
       if constexpr (MODE == SC_LAHQR) {
@@ -199,7 +200,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
           }
     }
     if constexpr (MODE == SC_FUSED || MODE == SC_TREVC) {
-      trevc_rows<P>(t, n, lane);
+      trevc_rows<P>(t, n, lane, top);
       __syncthreads();  // the eigenvector factor is ready
     }
   } else {
@@ -207,6 +208,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
     Rows z;
     z.init(lane);
     const int row0 = zi * Rows::RW, row = row0 + z.rl;
+    bool rare = false;  // an infinity or a NaN in the caller's rows
     if constexpr (MODE == SC_FUSED) {
       // the stages: the slots beside the one that the iteration is writing,
       // each as two vectors
@@ -218,6 +220,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
       for (int c = 0; c < SL; ++c) z.z[c] = mk<double>(SL * z.h + c == row ? 1.0 : 0.0, 0);
     } else {
       z.load(row, n, a.G, base, a.rB, a.iB);
+      rare = z.any_non_finite();
     }
     if constexpr (MODE == SC_LAHQR) {
       __syncthreads();  // the phases that made the subdiagonal real
@@ -231,7 +234,10 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
     }
     if constexpr (MODE == SC_FUSED || MODE == SC_TREVC) {
       __syncthreads();  // the eigenvector factor is ready
-      backtransform_mfma(t, z, row0, n, a.G, base, a.rB, a.iB);
+      if (MODE == SC_TREVC && rare)
+        backtransform_rare<P>(t, row0, min(row0 + Rows::RW, n), n, lane, a.G, base, a.rB, a.iB);
+      else
+        backtransform_mfma(t, z, row0, n, a.G, base, a.rB, a.iB);
     } else {
       z.store(row, n, a.G, base, a.rB, a.iB);
     }
