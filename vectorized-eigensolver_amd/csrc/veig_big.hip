@@ -293,6 +293,16 @@ int schur_for(const BigArgs &a, hipStream_t s) {
   // 64: 3.96 against 4.11 ms), past that the fewer wavefronts win
   if (a.G.n <= 80 && few_matrices(a.G, 2)) return launch_schur<20, 4, MODE>(a, s);
   if (a.G.n <= 80) return launch_schur<40, 2, MODE>(a, s);
+  // The stages load and store the rows of the caller, which 48 columns to a lane
+  // spill (1.9 KB of scratch against 0.3 with 24): ztrevc always takes the shorter
+  // segments (3,328 matrices, 48 -> 24 columns: order 81 4.01 -> 2.54 ms, 88 4.51 ->
+  // 2.89, 93 4.71 -> 3.16), zlahqr up to four matrices per CU (1,024: order 81 8.74
+  // -> 7.81 ms, 88 10.0 -> 9.1; 3,328: 28.6 -> 29.6, 32.7 -> 34.4) and where one
+  // matrix per CU is all that fits (order 94 x 3,328 63.5 -> 60.8), not where their
+  // longer ring is what leaves one (orders 90..93: 93 x 3,328 35.8 -> 59.5)
+  if constexpr (MODE == SC_TREVC) return launch_schur<24, 4, MODE>(a, s);
+  if constexpr (MODE == SC_LAHQR)
+    if (a.G.n > 93 || (a.G.n < 90 && few_matrices(a.G, 4))) return launch_schur<24, 4, MODE>(a, s);
   return launch_schur<48, 2, MODE>(a, s);
 }
 
