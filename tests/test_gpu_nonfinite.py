@@ -101,3 +101,19 @@ def test_eigenvectors_that_do_not_depend_on_it(gpu, n, bad):
         diff = np.abs(back(v, n)[0] - ref)
         assert np.all(diff[r, :j] <= tol * np.abs(ref).max())
         assert np.all(np.delete(diff, r, axis=0) <= tol * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("n", [33, 48, 64, 65, 80, 96])
+def test_infinite_first_diagonal_entry_deflates(gpu, n):
+    # H(1, 0) is negligible beside an infinite H(0, 0): the others are the eigenvalues of the rest
+    A = np.triu(H.gaussian(1, n, 9400 + n), -1)
+    for k in range(1, n):
+        A[0, k, k - 1] = abs(A[0, k, k - 1])
+    want = np.linalg.eigvals(A[0, 1:, 1:])
+    A[0, 0, 0] = np.inf
+    h, z, e = planes(A), planes(np.eye(n)[None] + 0j), zeros(n)
+    info = torch.full((1,), -1, dtype=torch.int32, device="cuda")
+    veig.zlahqr(n, 1, 1, *e, *h, *z, info=info)
+    assert int(info[0]) == 0
+    _, err = H.match_eigenvalues(want[None], vec(e, n)[:, 1:])
+    assert np.all(err <= 1e-11 * norm(A[:, 1:, 1:]))

@@ -622,8 +622,13 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
           const R ab = fmax(cabs1(h), cabs1(hup)), ba = fmin(cabs1(h), cabs1(hup));
           const R d3 = cabs1(sub(hkk1, hkk));
           const R aa = fmax(cabs1(hkk), d3), bb = fmin(cabs1(hkk), d3);
-          const R is = frcp(aa + ab);  // aa + ab >= cabs1(h) > 0
-          ng = ba * (ab * is) <= fmax(smlnum, ulp * (bb * (aa * is)));
+          const R s = aa + ab;  // >= cabs1(h) > 0
+          if constexpr (TZ) {
+            ng = ba * (ab / s) <= fmax(smlnum, ulp * (bb * (aa / s)));  // (s may be infinite)
+          } else {
+            const R is = frcp(s);
+            ng = ba * (ab * is) <= fmax(smlnum, ulp * (bb * (aa * is)));
+          }
         }
       }
       neg[p] = __ballot(ng);
