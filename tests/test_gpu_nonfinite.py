@@ -117,3 +117,46 @@ def test_infinite_first_diagonal_entry_deflates(gpu, n):
     assert int(info[0]) == 0
     _, err = H.match_eigenvalues(want[None], vec(e, n)[:, 1:])
     assert np.all(err <= 1e-11 * norm(A[:, 1:, 1:]))
+
+
+@pytest.mark.parametrize("bad", BAD)
+@pytest.mark.parametrize("n,m", [(n, m) for n in (33, 48, 64, 65, 80, 96) for m in (n // 2, 32, 24)] + [(16, 8), (24, 15)])
+def test_deflated_block_beside_an_undefined_one(gpu, n, m, bad):
+    # H(m, m-1) = 0: no rotation of the block from m on touches the columns
+    # before it, in T and in Z, and the eigenvalues there are theirs
+    A = np.triu(H.gaussian(1, n, 9500 + n), -1)
+    for k in range(1, n):
+        A[0, k, k - 1] = abs(A[0, k, k - 1])
+    A[0, m, m - 1] = 0
+    want = np.linalg.eigvals(A[0, :m, :m])
+    for r, c in ((m, m), (n - 1, n - 1), (0, m), (m - 1, m)):
+        B = A.copy()
+        B[0, r, c] = bad
+        h, z, e = planes(B), planes(np.eye(n)[None] + 0j), zeros(n)
+        veig.zlahqr(n, 1, 1, *e, *h, *z)
+        T, Z = back(h, n)[0], back(z, n)[0]
+        _, err = H.match_eigenvalues(want[None], vec(e, n)[:, :m])
+        assert np.all(err <= 1e-11 * norm(A[:, :m, :m]))
+        assert np.all(np.tril(T, -1) == 0)
+        R = A[0, :m, :m] @ Z[:m, :m] - Z[:m, :m] @ T[:m, :m]
+        assert norm(R) <= 1e-13 * n * norm(A[0, :m, :m])
+        assert np.all(Z[m:, :m] == 0)
+
+
+@pytest.mark.parametrize("bad", BAD)
+@pytest.mark.parametrize("n", [33, 48, 64, 65, 80, 96])
+def test_schur_vectors_beside_an_undefined_column(gpu, n, bad):
+    # diagonal but for one block: columns of Z outside it are copied
+    m = n // 2
+    A = np.diag(np.arange(1, n + 1) + 0j)[None].copy()
+    A[0, m:m + 3, m:m + 3] = np.triu(H.gaussian(1, 3, 9600 + n)[0], -1)
+    A[0, m + 1, m], A[0, m + 2, m + 1] = 1, 1
+    Z0 = H.gaussian(1, n, 9700 + n)
+    Z0[0, 0, m + 3], Z0[0, 1, m - 1], Z0[0, 2, n - 1], Z0[0, 3, m + 1] = bad, bad, bad, bad
+    h, z, e = planes(A), planes(Z0), zeros(n)
+    veig.zlahqr(n, 1, 1, *e, *h, *z)
+    Z = back(z, n)[0]
+    keep = np.r_[0:m, m + 3:n]
+    finite = np.isfinite(Z0[0][:, keep])
+    assert np.array_equal(Z[:, keep][finite], Z0[0][:, keep][finite])
+    assert np.all(np.isfinite(np.delete(Z[:, m:m + 3], 3, axis=0)))

@@ -177,6 +177,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
   if (w == hw) {
     // ---------------- the iteration and the eigenvector solve ----------------
     const unsigned top = wave_top(t.h, BandTile::entries(n), lane);
+    if (MODE == SC_LAHQR && lane == 0) ring.rare = top >= kNonFinite;  // (read after the next barrier)
     __builtin_amdgcn_s_setprio(3);  // the workgroup waits for the chain: it issues first on its SIMD
     if constexpr (MODE != SC_TREVC) {
       if constexpr (MODE == SC_LAHQR) {
@@ -208,7 +209,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
     Rows z;
     z.init(lane);
     const int row0 = zi * Rows::RW, row = row0 + z.rl;
-    bool rare = false;  // an infinity or a NaN in the caller's rows
+    bool rare = false;  // stages: an infinity or a NaN in the caller's matrix or rows
     if constexpr (MODE == SC_FUSED) {
       // the stages: the slots beside the one that the iteration is writing,
       // each as two vectors
@@ -228,16 +229,25 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
       for (int c = 0; c < SL; ++c)
         if (SL * z.h + c < n) z.z[c] = mulc(z.z[c], ld<double>(&ring.step[1][0].c + SL * z.h + c));
     }
-    if constexpr (MODE != SC_TREVC) {
-      z.start(ring, zi, zw);
-      z.replay(ring);
+    if constexpr (MODE != SC_TREVC) z.start(ring, zi, zw);
+    if constexpr (MODE == SC_LAHQR) rare = rare || __builtin_amdgcn_readfirstlane(ring.rare);
+    if constexpr (MODE == SC_LAHQR || MODE == SC_TREVC) {
+      if (__builtin_expect(rare, 0)) {  // the rest in the caller's planes
+        if constexpr (MODE == SC_LAHQR) {
+          z.store(row, n, a.G, base, a.rB, a.iB);
+          __threadfence_block();  // a row's segments, to the lane that takes it
+          replay_rare(&ring, lane < Rows::RW && row < n ? row : -1, a.G, base, a.rB, a.iB);
+        } else {
+          __syncthreads();  // the eigenvector factor is ready
+          backtransform_rare<P>(t, row0, min(row0 + Rows::RW, n), n, lane, a.G, base, a.rB, a.iB);
+        }
+        return;
+      }
     }
+    if constexpr (MODE != SC_TREVC) z.replay(ring);
     if constexpr (MODE == SC_FUSED || MODE == SC_TREVC) {
       __syncthreads();  // the eigenvector factor is ready
-      if (MODE == SC_TREVC && rare)
-        backtransform_rare<P>(t, row0, min(row0 + Rows::RW, n), n, lane, a.G, base, a.rB, a.iB);
-      else
-        backtransform_mfma(t, z, row0, n, a.G, base, a.rB, a.iB);
+      backtransform_mfma(t, z, row0, n, a.G, base, a.rB, a.iB);
     } else {
       z.store(row, n, a.G, base, a.rB, a.iB);
     }

@@ -29,10 +29,11 @@ namespace veig {
 
 // The Hessenberg part, row <= col + 1, column c from c(c+3)/2, or a dense
 // column-major tile.  Entries past the last are read (never used): kPad more
-// are allocated.
+// are allocated, the last of them to be written where a lane has nothing to write.
 struct BandTile {
   double2 *h;
   static constexpr int kPad = 2;
+  __device__ __forceinline__ double2 *spare(int n) const { return h + entries(n) - 1; }
   static __host__ __device__ constexpr int entries(int n) { return ((n - 1) * (n + 2)) / 2 + n + kPad; }
   static __device__ __forceinline__ int off(int c) { return (c * (c + 3)) >> 1; }
   static __device__ __forceinline__ int width(int c) { return c + 2; }  // off(c + 1) - off(c)
@@ -404,6 +405,7 @@ struct SweepRing {
   int L[R], I[R];  // steps L..I-1
   int last[R];
   int simd[8];     // chain_wave
+  int rare;        // the Hessenberg matrix holds an infinity or a NaN
 };
 // the record of a wavefront that keeps no Schur vectors: this sweep's r^2 only
 template <int CAP_>
@@ -677,8 +679,9 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
     x.hs = t.at(L + 2, L + 1)->x;  // past the last row: read and not used
 
     // ---- the sweep (Toolbox.hpp:138-335) ----
-    // the identity as the rotation before the first brings column L into the
-    // row updates and rewrites column L - 1 unchanged
+    // the identity as the rotation before the first, of (0, H(t, L)), brings
+    // column L into the row updates (of what is above the active block: column
+    // L - 1 may hold an infinity that column L does not, and the other way round)
     StreamLanes<P> a;
     a.q = Rot<R>{mk<R>(1, 0), 0.0};
     StepRec *rec = ring.step[slot];
@@ -692,9 +695,15 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
       a.t[p] = in ? t0 : I;
       const bool behind = a.t[p] < L;
       a.po[p] = behind ? t.at(at, L) : t.at(L, at) + 1;
-      a.pe[p] = a.po[p] - (behind ? T::width(L - 1) : 1);
+      a.pe[p] = a.po[p] - 1;
       a.e[p] = ld<R>(a.pe[p]);
       a.o[p] = ld<R>(a.po[p]);
+      if constexpr (TZ) {
+        if (behind) {
+          a.pe[p] = t.spare(n);
+          a.e[p] = mk<R>(0, 0);
+        }
+      }
       const int sc = t0 + 1 < I ? t0 + 1 : I - 1;
       a.sd[p] = t.at(sc + 1, sc)->x;
     }
@@ -974,6 +983,35 @@ struct SchurRows {
     }
   }
 };
+
+// SchurRows::replay where H or Z holds an infinity or a NaN: the steps of each
+// sweep alone, not the identity at the others, which would carry such a value
+// into the column beside it.  One lane to a row, in the output planes (row < 0:
+// none); as many barriers as replay.
+template <typename Ring>
+__device__ __noinline__ void replay_rare(const Ring *ring, int row, Geom G, int64_t base, double *re, double *im) {
+  for (int cur = 0;;) {
+    __syncthreads();
+    const int L = ring->L[cur], I = ring->I[cur];
+    if (row >= 0 && I > 0) {
+      auto put = [&](int c, cx<double> x) {
+        re[base + G.el(row, c)] = x.re;
+        im[base + G.el(row, c)] = x.im;
+      };
+      cx<double> z = mk<double>(re[base + G.el(row, L)], im[base + G.el(row, L)]);
+      for (int K = L; K < I; ++K) {
+        cx<double> next = mk<double>(re[base + G.el(row, K + 1)], im[base + G.el(row, K + 1)]);
+        rot_right(Rot<double>{ld<double>(&ring->step[cur][K].c), ring->step[cur][K].sr.x}, z, next);
+        put(K, z);
+        z = next;
+      }
+      put(I, mulc(z, ld<double>(&ring->ph[cur])));
+    }
+    const int last = __builtin_amdgcn_readfirstlane(ring->last[cur]);
+    cur = cur + 1 == Ring::R ? 0 : cur + 1;
+    if (last) return;
+  }
+}
 
 // --------------------------------------------------------------------------
 // Eigenvectors of the triangular tile (ztrevc + backsubstitution,
