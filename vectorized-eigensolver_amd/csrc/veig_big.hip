@@ -90,9 +90,9 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_reduce(BigA
     top = reduce_load(sm, n, a.G, base, a.rA, a.iA, top);
   } else {
     top = reduce_load(sm, n, a.G, base, a.rA, a.iA);
-    reduce_block(sm, n, top, tau);
+    const int e = reduce_block(sm, n, top, tau);
     const bool fused = MODE == RD_FUSED;
-    reduce_store(sm, n, a.G, base, fused ? a.rB : a.rA, fused ? a.iB : a.iA);
+    reduce_store(sm, n, a.G, base, fused ? a.rB : a.rA, fused ? a.iB : a.iA, e);
     if (a.rE && tid + 1 < n) {
       const cx<double> t = ld<double>(tau + tid);
       a.rE[vb + a.G.ve(tid)] = t.re;
@@ -178,6 +178,9 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
     // ---------------- the iteration and the eigenvector solve ----------------
     const unsigned top = wave_top(t.h, BandTile::entries(n), lane);
     if (MODE == SC_LAHQR && lane == 0) ring.rare = top >= kNonFinite;  // (read after the next barrier)
+    const int e2 = scale_exponent(top);  // (eigenvectors do not depend on it)
+    if (__builtin_expect(e2 != 0, 0)) scale_entries(t.h, BandTile::entries(n), lane, 64, e2);
+    lds_order();
     __builtin_amdgcn_s_setprio(3);  // the workgroup waits for the chain: it issues first on its SIMD
     if constexpr (MODE != SC_TREVC) {
       if constexpr (MODE == SC_LAHQR) {
@@ -186,7 +189,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
       }
       const int nfail = lahqr_stream<P, true>(t, n, lane, ring, a.itmax);
       for (int r = lane; r < n; r += 64) {
-        const cx<double> e = ld<double>(t.at(r, r));
+        const cx<double> e = cldexp(ld<double>(t.at(r, r)), e2);
         a.rE[vb + a.G.ve(r)] = e.re;
         a.iE[vb + a.G.ve(r)] = e.im;
       }
@@ -195,7 +198,7 @@ __global__ __launch_bounds__((schur_threads<SL, NT>())) __attribute__((amdgpu_wa
         for (int c = 0; c < n; ++c)
           for (int r = lane; r < n; r += 64) {
             const int64_t idx = base + a.G.el(r, c);
-            const cx<double> x = r <= c ? ld<double>(t.at(r, c)) : mk<double>(0, 0);
+            const cx<double> x = r <= c ? cldexp(ld<double>(t.at(r, c)), e2) : mk<double>(0, 0);
             a.rA[idx] = x.re;
             a.iA[idx] = x.im;
           }

@@ -176,7 +176,7 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_eig_block(E
   if (m >= a.G.nmat) return;  // workgroup-uniform
   const int n = a.G.n;
   const unsigned top = reduce_load(sm, n, a.G, a.G.mat_base(m), a.rA, a.iA);
-  reduce_block(sm, n, top, nullptr);
+  const int e2 = reduce_block(sm, n, top, nullptr);
   const int lane = threadIdx.x & 63;
   const DenseTile<S::LD> t{sm.H};
   auto &rec = *reinterpret_cast<SweepScratch<CAP> *>(sm.part);  // free now
@@ -185,7 +185,7 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_eig_block(E
     const int nfail = lahqr_stream<1, false>(t, n, lane, rec, a.itmax);
     const int64_t vb = a.G.vec_base(m);
     if (lane < n) {
-      const cx<double> e = ld<double>(t.at(lane, lane));
+      const cx<double> e = cldexp(ld<double>(t.at(lane, lane)), e2);
       a.rE[vb + a.G.ve(lane)] = e.re;
       a.iE[vb + a.G.ve(lane)] = e.im;
     }
@@ -218,9 +218,12 @@ __global__ __launch_bounds__(64) void k_eig_band(EigArgs a) {
       }
   }
   lds_order();
+  const int e2 = scale_exponent(wave_top(lds, BandTile::entries(n), lane));
+  if (__builtin_expect(e2 != 0, 0)) scale_entries(lds, BandTile::entries(n), lane, 64, e2);
+  lds_order();
   const int nfail = lahqr_stream<1, false>(t, n, lane, rec, a.itmax);
   if (lane < n) {
-    const cx<double> e = ld<double>(t.at(lane, lane));
+    const cx<double> e = cldexp(ld<double>(t.at(lane, lane)), e2);
     a.rE[vb + a.G.ve(lane)] = e.re;
     a.iE[vb + a.G.ve(lane)] = e.im;
   }
@@ -229,7 +232,7 @@ __global__ __launch_bounds__(64) void k_eig_band(EigArgs a) {
     for (int c = 0; c < n; ++c)
       if (lane <= c + 1 && lane < n) {
         const int64_t idx = base + a.G.el(lane, c);
-        const cx<double> h = ld<double>(t.at(lane, c));
+        const cx<double> h = cldexp(ld<double>(t.at(lane, c)), e2);
         a.rH[idx] = h.re;
         a.iH[idx] = h.im;
       }

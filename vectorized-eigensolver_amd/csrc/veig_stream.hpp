@@ -98,6 +98,25 @@ __device__ __forceinline__ unsigned high_word(double x) {
 }
 __device__ __forceinline__ unsigned high_word(cx<double> x) { return max(high_word(x.re), high_word(x.im)); }
 
+// The power of two that a matrix is divided by before its squares are formed, 0
+// where they fit as it is: with top (the largest high word) between 2^-300 and
+// 2^480 the sums of its squares stay finite, and the square of an entry 2^-150
+// times the largest stays normal.  Exact, so the results are those of the
+// unscaled matrix, scaled.
+__device__ __forceinline__ int scale_exponent(unsigned top) {
+  if (top >= kNonFinite) return 0;
+  const int e = (int)(top >> 20) - 1022;  // as frexp's (subnormal: -1022, small enough)
+  return e < -300 || e > 480 ? e : 0;
+}
+// a square below this is taken as zero: an entry below 2^-450, 2^-150 times the
+// largest at most, whose square is on the way to losing its bits
+constexpr double kTinySquare = 0x1p-900;
+
+// count entries of a tile divided by 2^e, by `threads` threads
+__device__ __forceinline__ void scale_entries(double2 *h, int count, int thread, int threads, int e) {
+  for (int i = thread; i < count; i += threads) st<double>(h + i, cldexp(ld<double>(h + i), -e));
+}
+
 // the largest high word over the wavefront's count entries
 __device__ __forceinline__ unsigned wave_top(const double2 *h, int count, int lane) {
   unsigned x = 0;
@@ -166,8 +185,9 @@ __device__ __forceinline__ void reduce_steps(ReduceBlock<CAP, W> &sm, int n, dou
     const cx<R> alpha = ld<R>(sm.at(i + 1, i));
     cx<R> tau = mk<R>(0, 0), scal = mk<R>(0, 0);
     R beta = alpha.re;
-    if (!(xnorm2 == 0.0 && alpha.im == 0.0)) {
-      const R nrm = fsqrt(abs2(alpha) + xnorm2);
+    const R nrm2 = abs2(alpha) + xnorm2;
+    if (!(xnorm2 == 0.0 && alpha.im == 0.0) && !(nrm2 < kTinySquare)) {
+      const R nrm = fsqrt(nrm2);
       beta = alpha.re >= 0.0 ? -nrm : nrm;
       const R ib = frcp(beta);
       tau = mk((beta - alpha.re) * ib, -alpha.im * ib);
@@ -259,11 +279,18 @@ __device__ __noinline__ void reduce_rare(ReduceBlock<CAP, W> *sm, int n, double2
   reduce_steps<true>(*sm, n, tau_out);
 }
 
-// top: the largest high word of the input, from reduce_load
+// top: the largest high word of the input, from reduce_load.  Returns the e of
+// the 2^e that the tile's H is divided by (scale_exponent).
 template <int CAP, int W>
-__device__ __forceinline__ void reduce_block(ReduceBlock<CAP, W> &sm, int n, unsigned top, double2 *tau_out) {
+__device__ __forceinline__ int reduce_block(ReduceBlock<CAP, W> &sm, int n, unsigned top, double2 *tau_out) {
+  const int e = scale_exponent(top);
+  if (__builtin_expect(e != 0, 0)) {
+    scale_entries(sm.H, (int)(sizeof(sm.H) / sizeof(double2)), threadIdx.x, blockDim.x, e);
+    __syncthreads();
+  }
   if (__builtin_expect(top >= kNonFinite, 0)) reduce_rare(&sm, n, tau_out);
   else reduce_steps<false>(sm, n, tau_out);
+  return e;
 }
 
 // the tile from memory, zeros outside the matrix (ends at a barrier); returns
@@ -294,10 +321,10 @@ __device__ __forceinline__ unsigned reduce_load(ReduceBlock<CAP, W> &sm, int n, 
   return block_max(top, sm.words);
 }
 
-// the tile to memory
+// the tile to memory, H times 2^e (the reflectors below its subdiagonal as they are)
 template <int CAP, int W>
 __device__ __forceinline__ void reduce_store(ReduceBlock<CAP, W> &sm, int n, const Geom &G, int64_t base, double *re,
-                                             double *im) {
+                                             double *im, int e) {
   constexpr int CH = ReduceBlock<CAP, W>::CH;
   const int r = threadIdx.x % CAP, q = threadIdx.x / CAP;
 #pragma unroll
@@ -305,7 +332,7 @@ __device__ __forceinline__ void reduce_store(ReduceBlock<CAP, W> &sm, int n, con
     const int c = q * CH + j;
     if (q < W && r < n && c < n) {
       const int64_t idx = base + G.el(r, c);
-      const cx<double> x = ld<double>(sm.at(r, c));
+      const cx<double> x = cldexp(ld<double>(sm.at(r, c)), r <= c + 1 ? e : 0);
       re[idx] = x.re;
       im[idx] = x.im;
     }
@@ -497,11 +524,11 @@ struct StreamWindow {
   uint64_t none, none_hi;  // bit K (K - 64): step K's input was zero, its rotation the identity
   cx<double> was;       // a0 where the last one was replaced
 
-  // m2, and the zero vector (or one below the underflow threshold) replaced
+  // m2, and the zero vector (or one below kTinySquare) replaced
   // by one that gives G = I
   __device__ __forceinline__ void norm(int K) {
     m2 = fma(a0.re, a0.re, fma(a0.im, a0.im, a1 * a1));
-    if (__builtin_expect(__any(m2 == 0.0), 0)) {
+    if (__builtin_expect(__any(m2 < kTinySquare), 0)) {
       was = a0;
       a0 = mk<double>(1, 0);
       a1 = 0.0;
@@ -742,7 +769,7 @@ __device__ __forceinline__ int lahqr_stream(const T &t, int n, int lane, RING &r
     // on the way out: row I right of I and column I above it scaled
     cx<R> zz = mk<R>(1, 0);
     cx<R> hsub = ((I < 64 ? x.none : x.none_hi) >> (I & 63)) & 1u ? x.was : x.a0;
-    if (hsub.im != 0.0 && abs2(hsub) > 0.0) {  // |h|^2 may underflow: leave such h alone
+    if (hsub.im != 0.0 && abs2(hsub) > kTinySquare) {  // a smaller h: negligible, or its real part is taken
       const R m2 = abs2(hsub), id = frsq(m2);
       zz = mk(hsub.re * id, -hsub.im * id);  // conj(h/|h|)
       hsub = mk(m2 * id, 0.0);
