@@ -77,12 +77,15 @@ def build_lib(verbose: bool = False) -> Path:
 
 
 def build_probes(verbose: bool = False) -> None:
-    """The test probe of the scalar complex API (include/veig_complex.hpp):
-    a host build (g++) and a gfx950 build (hipcc) of tests/probe/."""
+    """The test probes in tests/probe/: the scalar complex API
+    (include/veig_complex.hpp) in a host build (g++) and a gfx950 build
+    (hipcc), and the choice of the chain's wavefront (host)."""
     probe = REPO / "tests" / "probe"
     cmds = [
         ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", str(REPO / "include"),
          "-o", str(probe / "libcomplex_probe_host.so"), str(probe / "complex_probe_host.cpp")],
+        ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-I", str(CSRC),
+         "-o", str(probe / "libchain_probe_host.so"), str(probe / "chain_probe_host.cpp")],
         [hipcc(), *HIPCC_FLAGS, "-I", str(REPO / "include"),
          "-o", str(probe / "libcomplex_probe.so"), str(probe / "complex_probe.hip")],
     ]

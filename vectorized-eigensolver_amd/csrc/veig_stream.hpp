@@ -23,6 +23,7 @@
 // rotate), so each update is one load and one store per lane instead of two
 // of each, and none of them is on the chain.
 #pragma once
+#include "veig_chain.hpp"
 #include "veig_common.hpp"
 
 namespace veig {
@@ -58,29 +59,17 @@ __device__ __forceinline__ double read_lane(double x, int lane) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
-// The wavefront of the workgroup that runs the chain.  Of the workgroups that
-// share a CU each should have its chain on another SIMD: two chains on one
-// SIMD take nearly twice as long.  Four workgroups of three wavefronts, three
-// to a SIMD, leave each SIMD out once, and a workgroup that takes an ended
-// one's place takes its SIMDs: the SIMD after the one left out is another one
-// in each.  Wider workgroups have a wavefront on every SIMD: there the
-// workgroup's place in the CU's LDS numbers it among its neighbours.  ids:
-// one LDS word per wavefront.  Every thread calls it (one barrier).
+// The wavefront of the workgroup that runs the chain (chain_pick), the same in
+// every wavefront.  ids: one LDS word per wavefront.  Every thread calls it (one
+// barrier).
 __device__ __forceinline__ int chain_wave(int *ids) {
   constexpr int kHwId = 4, kLdsAlloc = 6;  // hardware registers, read whole (32 bits from bit 0)
-  const unsigned simd = (__builtin_amdgcn_s_getreg((31 << 11) | kHwId) >> 4) & 3u;
+  const unsigned hw = __builtin_amdgcn_s_getreg((31 << 11) | kHwId);
   const unsigned lds = __builtin_amdgcn_s_getreg((31 << 11) | kLdsAlloc);
-  const unsigned base = lds & 0xfffu, size = (lds >> 12) & 0xfffu;
-  const int waves = blockDim.x >> 6;
-  if ((threadIdx.x & 63) == 0) ids[threadIdx.x >> 6] = (int)simd;
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) ids[wave] = chain_note(wave, hw, lds);
   __syncthreads();
-  unsigned there = 0;
-  for (int w = 0; w < waves; ++w) there |= 1u << (ids[w] & 3);
-  const unsigned want = there == 15u ? (size ? base / size : 0u) : (unsigned)__builtin_ctz(~there) + 1u;
-  for (unsigned d = 0; d < 4; ++d)
-    for (int w = 0; w < waves; ++w)
-      if (((unsigned)ids[w] & 3u) == ((want + d) & 3u)) return __builtin_amdgcn_readfirstlane(w);
-  return 0;
+  return __builtin_amdgcn_readfirstlane(chain_pick(ids, blockDim.x >> 6));
 }
 
 // sum over the wavefront, the same bits in every lane: rows of 16 by DPP, the
