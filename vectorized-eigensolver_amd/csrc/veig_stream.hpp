@@ -261,8 +261,13 @@ __device__ __forceinline__ void reduce_steps(ReduceBlock<CAP, W> &sm, int n, dou
   }
 }
 
-// (a call: inlined, it cost the usual input's kernels 1 to 3%, in registers and
+// (calls: inlined, they cost the usual input's kernels 1 to 3%, in registers and
 // in the order that the rest came out in)
+template <int CAP, int W>
+__device__ __noinline__ void scale_block(ReduceBlock<CAP, W> *sm, int e) {
+  scale_entries(sm->H, (int)(sizeof(sm->H) / sizeof(double2)), threadIdx.x, blockDim.x, e);
+  __syncthreads();
+}
 template <int CAP, int W>
 __device__ __noinline__ void reduce_rare(ReduceBlock<CAP, W> *sm, int n, double2 *tau_out) {
   reduce_steps<true>(*sm, n, tau_out);
@@ -274,8 +279,7 @@ template <int CAP, int W>
 __device__ __forceinline__ int reduce_block(ReduceBlock<CAP, W> &sm, int n, unsigned top, double2 *tau_out) {
   const int e = scale_exponent(top);
   if (__builtin_expect(e != 0, 0)) {
-    scale_entries(sm.H, (int)(sizeof(sm.H) / sizeof(double2)), threadIdx.x, blockDim.x, e);
-    __syncthreads();
+    scale_block(&sm, e);
   }
   if (__builtin_expect(top >= kNonFinite, 0)) reduce_rare(&sm, n, tau_out);
   else reduce_steps<false>(sm, n, tau_out);
