@@ -18,6 +18,13 @@
  *                (utils.h:37-65); they allocate device memory, copy in, run the
  *                device entry and copy back, like utils.cpp:631-692, and return
  *                after the results are on the host.
+ * The kernels of an entry are chosen by order and by number of matrices (batches
+ * too small to fill the GPU, orders 4..32, take others; orders 65..93 by
+ * how many share a compute unit).  They differ in the order of their operations, so the
+ * same matrix in a batch of another size may come out with other last bits, and
+ * where rounding decides which eigenvalue deflates first, with E and the columns
+ * of V in another order and of another length.  One size gives one result; the
+ * per-matrix entries of veig_compat.hpp follow the batch they are told of.
  * Every function returns a veig_status; veig_last_error() describes the last
  * failure of the calling thread.  Sizes are 64-bit (the reference's 32-bit
  * int byte counts overflow at 2^31 bytes per plane).

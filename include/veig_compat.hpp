@@ -102,11 +102,12 @@ void test_backsubstitution(double *rT, double *iT, double *rx, double *ix, int d
 // 1133): ONE matrix of the tiled layout, the pointers pre-offset to its slot
 // and its elements thread_cnt apart (element (r, c) of the dim x dim matrix
 // at p[(r + c*dim) * thread_cnt], vector entry i at p[i * thread_cnt]), as
-// the batch entries above pass them.  Each call gathers the matrix, runs the
-// batch entry on it as a batch of one on the GPU and scatters the results
-// back, so its values are the batch entry's for that slot; a caller that
-// loops over slots should call the batch entry instead (one launch instead
-// of one per matrix).  The work arrays are accepted and unused.
+// the batch entries above pass them.  Each call gathers the matrix, runs it
+// on the GPU through the kernels that the batch entry takes for block_cnt *
+// thread_cnt matrices and scatters the results back, so its values are the
+// batch entry's for that slot; a caller that loops over slots should call the
+// batch entry instead (one launch instead of one per matrix).  The work arrays
+// are accepted and unused.
 void zgehrd(double *rA, double *iA, double *rtau, double *itau, double *rwork, double *iwork, int dim,
             int block_cnt, int thread_cnt);
 void zunghr(double *rA, double *iA, double *rtau, double *itau, double *rwork, double *iwork, int dim,

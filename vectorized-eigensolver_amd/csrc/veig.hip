@@ -10,6 +10,7 @@
 #include <string>
 
 #include "veig_common.hpp"
+#include "veig_slot.hpp"
 
 namespace veig {
 std::string &last_error() {
@@ -45,12 +46,13 @@ enum { ST_GEHRD = 0, ST_HESS = 1, ST_UNGHR = 2, ST_LAHQR = 3, ST_TREVC = 4 };
 // 2.25 ms, 24 4.42 -> 3.01, 32 7.03 -> 4.00; ztrevc 1.11 -> 0.95, 1.92 -> 1.49,
 // 2.88 -> 2.27; at order 16 they lose, 0.65 -> 0.71 and 0.33 -> 0.73).  Below
 // it the reduction does up to four matrices per CU (order 16 x 1,024: 68 ->
-// 44 us), the QR iteration up to one (few_matrices).
-bool per_workgroup(int mode, const Geom &G) {
-  if (G.n > 32) return true;
-  if (mode == ST_LAHQR) return G.n >= 8 && few_matrices(G, 1);
-  if (G.n > 16) return true;
-  return mode != ST_TREVC && G.n >= 8 && few_matrices(G, 4);
+// 44 us), the QR iteration up to one (few_matrices).  batch: the matrices of
+// the batch, or of the one that a single matrix is taken out of (veig_slot.hpp).
+bool per_workgroup(int mode, int n, int64_t batch) {
+  if (n > 32) return true;
+  if (mode == ST_LAHQR) return n >= 8 && few_matrices(batch, 1);
+  if (n > 16) return true;
+  return mode != ST_TREVC && n >= 8 && few_matrices(batch, 4);
 }
 
 template <int NB>
@@ -240,7 +242,25 @@ int launch_stage(const StageArgs &a, hipStream_t s) {
   return VEIG_OK;
 }
 
-
+int stage_zgehrd(const Geom &G, int64_t batch, double *rA, double *iA, double *rtau, double *itau, hipStream_t s) {
+  if (per_workgroup(ST_GEHRD, G.n, batch)) return launch_big(BIG_GEHRD, G, rA, iA, nullptr, nullptr, rtau, itau, nullptr, 30, 0, s);
+  return launch_stage(StageArgs{rA, iA, nullptr, nullptr, rtau, itau, nullptr, G, 30, ST_GEHRD}, s);
+}
+int stage_zunghr(const Geom &G, int64_t batch, double *rA, double *iA, double *rtau, double *itau, hipStream_t s) {
+  if (per_workgroup(ST_UNGHR, G.n, batch)) return launch_big(BIG_UNGHR, G, rA, iA, nullptr, nullptr, rtau, itau, nullptr, 30, 0, s);
+  return launch_stage(StageArgs{rA, iA, nullptr, nullptr, rtau, itau, nullptr, G, 30, ST_UNGHR}, s);
+}
+int stage_zlahqr(const Geom &G, int64_t batch, double *rE, double *iE, double *rH, double *iH, double *rZ, double *iZ,
+                 int32_t *info, int itmax, hipStream_t s) {
+  if (per_workgroup(ST_LAHQR, G.n, batch))
+    return launch_big(BIG_LAHQR, G, rH, iH, rZ, iZ, rE, iE, info, itmax, 0, s, nullptr, nullptr, nullptr, nullptr, batch);
+  return launch_stage(StageArgs{rH, iH, rZ, iZ, rE, iE, info, G, itmax, ST_LAHQR}, s);
+}
+int stage_ztrevc(const Geom &G, int64_t batch, double *rT, double *iT, double *rR, double *iR, hipStream_t s) {
+  if (per_workgroup(ST_TREVC, G.n, batch))
+    return launch_big(BIG_TREVC, G, rT, iT, rR, iR, nullptr, nullptr, nullptr, 30, 0, s, nullptr, nullptr, nullptr, nullptr, batch);
+  return launch_stage(StageArgs{rT, iT, rR, iR, nullptr, nullptr, nullptr, G, 30, ST_TREVC}, s);
+}
 
 // RAII device buffer for the host mirrors
 struct DevBuf {
@@ -266,6 +286,63 @@ int d2h(double *h, const DevBuf &b, size_t count) {
 }
 
 }  // namespace
+
+// ============================================================================
+// one matrix, as a batch takes it
+// ============================================================================
+namespace veig {
+
+int slot_zgehrd(int dim, int64_t batch, double *rA, double *iA, double *rtau, double *itau) {
+  VEIG_TRY(check_geom(dim, 1, 1));
+  const size_t sv = (size_t)dim, sm = sv * dim;
+  DevBuf a, b, t, u;
+  VEIG_TRY(dev_alloc(a, sm)); VEIG_TRY(dev_alloc(b, sm)); VEIG_TRY(dev_alloc(t, sv)); VEIG_TRY(dev_alloc(u, sv));
+  VEIG_TRY(h2d(a, rA, sm)); VEIG_TRY(h2d(b, iA, sm)); VEIG_TRY(h2d(t, rtau, sv)); VEIG_TRY(h2d(u, itau, sv));
+  VEIG_TRY(stage_zgehrd(make_geom(dim, 1, 1), batch, a.p, b.p, t.p, u.p, nullptr));
+  VEIG_HIP(hipDeviceSynchronize());
+  VEIG_TRY(d2h(rA, a, sm)); VEIG_TRY(d2h(iA, b, sm)); VEIG_TRY(d2h(rtau, t, sv)); VEIG_TRY(d2h(itau, u, sv));
+  return VEIG_OK;
+}
+
+int slot_zunghr(int dim, int64_t batch, double *rA, double *iA, double *rtau, double *itau) {
+  VEIG_TRY(check_geom(dim, 1, 1));
+  const size_t sv = (size_t)dim, sm = sv * dim;
+  DevBuf a, b, t, u;
+  VEIG_TRY(dev_alloc(a, sm)); VEIG_TRY(dev_alloc(b, sm)); VEIG_TRY(dev_alloc(t, sv)); VEIG_TRY(dev_alloc(u, sv));
+  VEIG_TRY(h2d(a, rA, sm)); VEIG_TRY(h2d(b, iA, sm)); VEIG_TRY(h2d(t, rtau, sv)); VEIG_TRY(h2d(u, itau, sv));
+  VEIG_TRY(stage_zunghr(make_geom(dim, 1, 1), batch, a.p, b.p, t.p, u.p, nullptr));
+  VEIG_HIP(hipDeviceSynchronize());
+  VEIG_TRY(d2h(rA, a, sm)); VEIG_TRY(d2h(iA, b, sm));
+  return VEIG_OK;
+}
+
+int slot_zlahqr(int dim, int64_t batch, double *rE, double *iE, double *rH, double *iH, double *rZ, double *iZ) {
+  VEIG_TRY(check_geom(dim, 1, 1));
+  const size_t sv = (size_t)dim, sm = sv * dim;
+  DevBuf e, f, a, b, s, u;
+  VEIG_TRY(dev_alloc(e, sv)); VEIG_TRY(dev_alloc(f, sv)); VEIG_TRY(dev_alloc(a, sm)); VEIG_TRY(dev_alloc(b, sm));
+  VEIG_TRY(dev_alloc(s, sm)); VEIG_TRY(dev_alloc(u, sm));
+  VEIG_TRY(h2d(a, rH, sm)); VEIG_TRY(h2d(b, iH, sm)); VEIG_TRY(h2d(s, rZ, sm)); VEIG_TRY(h2d(u, iZ, sm));
+  VEIG_TRY(stage_zlahqr(make_geom(dim, 1, 1), batch, e.p, f.p, a.p, b.p, s.p, u.p, nullptr, 30, nullptr));
+  VEIG_HIP(hipDeviceSynchronize());
+  VEIG_TRY(d2h(rE, e, sv)); VEIG_TRY(d2h(iE, f, sv)); VEIG_TRY(d2h(rH, a, sm)); VEIG_TRY(d2h(iH, b, sm));
+  VEIG_TRY(d2h(rZ, s, sm)); VEIG_TRY(d2h(iZ, u, sm));
+  return VEIG_OK;
+}
+
+int slot_ztrevc(int dim, int64_t batch, double *rT, double *iT, double *rR, double *iR) {
+  VEIG_TRY(check_geom(dim, 1, 1));
+  const size_t sm = (size_t)dim * dim;
+  DevBuf a, b, c, d;
+  VEIG_TRY(dev_alloc(a, sm)); VEIG_TRY(dev_alloc(b, sm)); VEIG_TRY(dev_alloc(c, sm)); VEIG_TRY(dev_alloc(d, sm));
+  VEIG_TRY(h2d(a, rT, sm)); VEIG_TRY(h2d(b, iT, sm)); VEIG_TRY(h2d(c, rR, sm)); VEIG_TRY(h2d(d, iR, sm));
+  VEIG_TRY(stage_ztrevc(make_geom(dim, 1, 1), batch, a.p, b.p, c.p, d.p, nullptr));
+  VEIG_HIP(hipDeviceSynchronize());
+  VEIG_TRY(d2h(rR, c, sm)); VEIG_TRY(d2h(iR, d, sm));
+  return VEIG_OK;
+}
+
+}  // namespace veig
 
 // ============================================================================
 // C ABI
@@ -315,9 +392,7 @@ int veig_zgehrd(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rA, 
   if (empty_batch(dim, block_cnt, thread_cnt)) return VEIG_OK;
   VEIG_REQUIRE(rA); VEIG_REQUIRE(iA); VEIG_REQUIRE(rtau); VEIG_REQUIRE(itau);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
-  if (per_workgroup(ST_GEHRD, G)) return launch_big(BIG_GEHRD, G, rA, iA, nullptr, nullptr, rtau, itau, nullptr, 30, 0, (hipStream_t)stream);
-  StageArgs a{rA, iA, nullptr, nullptr, rtau, itau, nullptr, G, 30, ST_GEHRD};
-  return launch_stage(a, (hipStream_t)stream);
+  return stage_zgehrd(G, G.nmat, rA, iA, rtau, itau, (hipStream_t)stream);
 }
 
 int veig_hessenberg(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rA, double *iA,
@@ -328,7 +403,7 @@ int veig_hessenberg(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *
   // tau is produced and consumed on chip (Q is accumulated forward), so no
   // tau planes are needed: the kernels skip writing it
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
-  if (per_workgroup(ST_HESS, G)) return launch_big(BIG_HESS, G, rA, iA, rQ, iQ, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
+  if (per_workgroup(ST_HESS, G.n, G.nmat)) return launch_big(BIG_HESS, G, rA, iA, rQ, iQ, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
   StageArgs a{rA, iA, rQ, iQ, nullptr, nullptr, nullptr, G, 30, ST_HESS};
   return launch_stage(a, (hipStream_t)stream);
 }
@@ -340,9 +415,7 @@ int veig_zunghr(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rA, 
   VEIG_REQUIRE(rA); VEIG_REQUIRE(iA); VEIG_REQUIRE(rtau); VEIG_REQUIRE(itau);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
   double *rt = const_cast<double *>(rtau), *it = const_cast<double *>(itau);
-  if (per_workgroup(ST_UNGHR, G)) return launch_big(BIG_UNGHR, G, rA, iA, nullptr, nullptr, rt, it, nullptr, 30, 0, (hipStream_t)stream);
-  StageArgs a{rA, iA, nullptr, nullptr, rt, it, nullptr, G, 30, ST_UNGHR};
-  return launch_stage(a, (hipStream_t)stream);
+  return stage_zunghr(G, G.nmat, rA, iA, rt, it, (hipStream_t)stream);
 }
 
 int veig_zlahqr(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rE, double *iE,
@@ -352,10 +425,7 @@ int veig_zlahqr(int64_t dim, int64_t block_cnt, int64_t thread_cnt, double *rE, 
   if (empty_batch(dim, block_cnt, thread_cnt)) return VEIG_OK;
   VEIG_REQUIRE(rE); VEIG_REQUIRE(iE); VEIG_REQUIRE(rH); VEIG_REQUIRE(iH); VEIG_REQUIRE(rZ); VEIG_REQUIRE(iZ);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
-  const int its = itmax > 0 ? itmax : 30;
-  if (per_workgroup(ST_LAHQR, G)) return launch_big(BIG_LAHQR, G, rH, iH, rZ, iZ, rE, iE, info, its, 0, (hipStream_t)stream);
-  StageArgs a{rH, iH, rZ, iZ, rE, iE, info, G, its, ST_LAHQR};
-  return launch_stage(a, (hipStream_t)stream);
+  return stage_zlahqr(G, G.nmat, rE, iE, rH, iH, rZ, iZ, info, itmax > 0 ? itmax : 30, (hipStream_t)stream);
 }
 
 int veig_ztrevc(int64_t dim, int64_t block_cnt, int64_t thread_cnt, const double *rT,
@@ -365,9 +435,7 @@ int veig_ztrevc(int64_t dim, int64_t block_cnt, int64_t thread_cnt, const double
   VEIG_REQUIRE(rT); VEIG_REQUIRE(iT); VEIG_REQUIRE(rR); VEIG_REQUIRE(iR);
   const Geom G = make_geom(dim, block_cnt, thread_cnt);
   double *rt = const_cast<double *>(rT), *it = const_cast<double *>(iT);
-  if (per_workgroup(ST_TREVC, G)) return launch_big(BIG_TREVC, G, rt, it, rR, iR, nullptr, nullptr, nullptr, 30, 0, (hipStream_t)stream);
-  StageArgs a{rt, it, rR, iR, nullptr, nullptr, nullptr, G, 30, ST_TREVC};
-  return launch_stage(a, (hipStream_t)stream);
+  return stage_ztrevc(G, G.nmat, rt, it, rR, iR, (hipStream_t)stream);
 }
 
 int veig_zgemv(int hermitian, int64_t dim, int64_t block_cnt, int64_t thread_cnt,

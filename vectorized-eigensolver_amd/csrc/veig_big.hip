@@ -297,14 +297,14 @@ int launch_schur(const BigArgs &a, hipStream_t s) {
 }
 
 template <int MODE>
-int schur_for(const BigArgs &a, hipStream_t s) {
+int schur_for(const BigArgs &a, hipStream_t s, int64_t batch) {
   if (a.G.n <= 32) return launch_schur<16, 2, MODE>(a, s);
   if (a.G.n <= 40) return launch_schur<20, 2, MODE>(a, s);
   if (a.G.n <= 48) return launch_schur<24, 2, MODE>(a, s);
   if (a.G.n <= 64) return launch_schur<32, 2, MODE>(a, s);
   // two matrices per CU at most: the shorter segments replay sooner (order 79 x
   // 64: 3.96 against 4.11 ms), past that the fewer wavefronts win
-  if (a.G.n <= 80 && few_matrices(a.G, 2)) return launch_schur<20, 4, MODE>(a, s);
+  if (a.G.n <= 80 && few_matrices(batch, 2)) return launch_schur<20, 4, MODE>(a, s);
   if (a.G.n <= 80) return launch_schur<40, 2, MODE>(a, s);
   // The stages load and store the rows of the caller, which 48 columns to a lane
   // spill (1.9 KB of scratch against 0.3 with 24): ztrevc always takes the shorter
@@ -315,7 +315,7 @@ int schur_for(const BigArgs &a, hipStream_t s) {
   // longer ring is what leaves one (orders 90..93: 93 x 3,328 35.8 -> 59.5)
   if constexpr (MODE == SC_TREVC) return launch_schur<24, 4, MODE>(a, s);
   if constexpr (MODE == SC_LAHQR)
-    if (a.G.n > 93 || (a.G.n < 90 && few_matrices(a.G, 4))) return launch_schur<24, 4, MODE>(a, s);
+    if (a.G.n > 93 || (a.G.n < 90 && few_matrices(batch, 4))) return launch_schur<24, 4, MODE>(a, s);
   return launch_schur<48, 2, MODE>(a, s);
 }
 
@@ -325,20 +325,21 @@ namespace veig {
 
 int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, double *iB, double *rE, double *iE,
                int32_t *info, int itmax, uint32_t flags, hipStream_t s, const int32_t *list,
-               const int32_t *list_count, const double *rC, const double *iC) {
+               const int32_t *list_count, const double *rC, const double *iC, int64_t batch) {
   if (G.n > VEIG_MAX_DIM) return fail(VEIG_ERR_UNSUPPORTED, "order beyond VEIG_MAX_DIM");
   if (G.nmat > INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");
   const BigArgs a{rA, iA, rB, iB, rE, iE, info, G, itmax > 0 ? itmax : 30, flags, list, list_count, rC, iC};
+  if (!batch) batch = G.nmat;
   switch (mode) {
     case BIG_FUSED:
       VEIG_TRY(reduce_for<RD_FUSED>(a, s));
-      return schur_for<SC_FUSED>(a, s);
+      return schur_for<SC_FUSED>(a, s, batch);
     case BIG_REDUCE: return reduce_for<RD_FUSED>(a, s);
     case BIG_GEHRD: return reduce_for<RD_GEHRD>(a, s);
     case BIG_HESS: return reduce_for<RD_HESS>(a, s);
     case BIG_UNGHR: return reduce_for<RD_UNGHR>(a, s);
-    case BIG_LAHQR: return schur_for<SC_LAHQR>(a, s);
-    case BIG_TREVC: return schur_for<SC_TREVC>(a, s);
+    case BIG_LAHQR: return schur_for<SC_LAHQR>(a, s, batch);
+    case BIG_TREVC: return schur_for<SC_TREVC>(a, s, batch);
     default:  // BIG_ROOTS: orders up to VEIG_MAX_DIM_FAST
       return G.n <= 48 ? launch_schur<24, 2, SC_ROOTS>(a, s) : launch_schur<32, 2, SC_ROOTS>(a, s);
   }

@@ -399,11 +399,13 @@ int launch_zgeev64(const FusedArgs &a, hipStream_t s);
 // zunghr (reflectors in A, tau in E -> Q in A), zlahqr (H in A -> T, Z in B
 // updated, E), ztrevc (T in A, B <- B X); polynomial roots with their Schur
 // form (coefficients in C -> T in A, Z in B, E); the fused path's reduction
-// alone, for the banded kernels (A -> compact form in B, tau in E).
+// alone, for the banded kernels (A -> compact form in B, tau in E).  batch: the
+// kernels are chosen as for so many matrices (0: for the batch's).
 enum { BIG_FUSED = 0, BIG_GEHRD = 1, BIG_HESS = 2, BIG_UNGHR = 3, BIG_LAHQR = 4, BIG_TREVC = 5, BIG_ROOTS = 6, BIG_REDUCE = 7 };
 int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, double *iB, double *rE, double *iE,
                int32_t *info, int itmax, uint32_t flags, hipStream_t s, const int32_t *list = nullptr,
-               const int32_t *list_count = nullptr, const double *rC = nullptr, const double *iC = nullptr);
+               const int32_t *list_count = nullptr, const double *rC = nullptr, const double *iC = nullptr,
+               int64_t batch = 0);
 
 // Batches too small to fill the chip with lane groups go to the
 // one-matrix-per-workgroup kernels (veig_stream.hpp), whose single matrix is
@@ -425,7 +427,8 @@ int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, doub
 // so one per CU with Schur vectors, four without (eigvals above order 16: one,
 // its dense tile letting fewer workgroups share a CU).
 constexpr int64_t kComputeUnits = 256;  // MI355X
-inline bool few_matrices(const Geom &G, int per_cu) { return G.nmat <= per_cu * kComputeUnits; }
+inline bool few_matrices(int64_t nmat, int per_cu) { return nmat <= per_cu * kComputeUnits; }
+inline bool few_matrices(const Geom &G, int per_cu) { return few_matrices(G.nmat, per_cu); }
 
 // FP64 batches and lists of orders up to NB on lane groups of LW lanes
 // (0: NB): Hessenberg reduction, then the QR iteration and eigenvectors on

@@ -3,6 +3,8 @@
 // include/veig_compat.hpp for the semantics.
 #include "veig_compat.hpp"
 
+#include "veig_slot.hpp"
+
 #include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
@@ -285,27 +287,32 @@ bool slot_args(int dim, int thread_cnt, const char *what) {
   if (thread_cnt <= 0) throw veig::Error(VEIG_ERR_INVALID, std::string(what) + ": thread_cnt must be positive");
   return dim > 0;  // an empty matrix: nothing to do, as in the reference
 }
+
+// the matrices of the batch that the slot is one of
+int64_t slot_batch(int block_cnt, int thread_cnt) { return (int64_t)(block_cnt > 0 ? block_cnt : 1) * thread_cnt; }
 }  // namespace
 
-void zgehrd(double *rA, double *iA, double *rtau, double *itau, double *, double *, int dim, int,
+void zgehrd(double *rA, double *iA, double *rtau, double *itau, double *, double *, int dim, int block_cnt,
             int thread_cnt) {
   if (!slot_args(dim, thread_cnt, "zgehrd")) return;
   Slot a(rA, iA, (size_t)dim * dim, thread_cnt, "zgehrd"), t(rtau, itau, (size_t)dim, thread_cnt, "zgehrd");
-  call_zgehrd(dim, 1, 1, a.re.data(), a.im.data(), t.re.data(), t.im.data());
+  check(veig::slot_zgehrd(dim, slot_batch(block_cnt, thread_cnt), a.re.data(), a.im.data(), t.re.data(), t.im.data()),
+        "zgehrd");
   a.back();
   t.back();
 }
 
-void zunghr(double *rA, double *iA, double *rtau, double *itau, double *, double *, int dim, int,
+void zunghr(double *rA, double *iA, double *rtau, double *itau, double *, double *, int dim, int block_cnt,
             int thread_cnt) {
   if (!slot_args(dim, thread_cnt, "zunghr")) return;
   Slot a(rA, iA, (size_t)dim * dim, thread_cnt, "zunghr"), t(rtau, itau, (size_t)dim, thread_cnt, "zunghr");
-  call_zunghr(dim, 1, 1, a.re.data(), a.im.data(), t.re.data(), t.im.data());
+  check(veig::slot_zunghr(dim, slot_batch(block_cnt, thread_cnt), a.re.data(), a.im.data(), t.re.data(), t.im.data()),
+        "zunghr");
   a.back();
 }
 
 void zlahqr_schur(bool, bool wantZ, int dim, double *rV, double *iV, double *rE, double *iE, double *rZ,
-                  double *iZ, int, int thread_cnt) {
+                  double *iZ, int block_cnt, int thread_cnt) {
   if (!slot_args(dim, thread_cnt, "zlahqr_schur")) return;
   const size_t nn = (size_t)dim * dim;
   Slot v(rV, iV, nn, thread_cnt, "zlahqr_schur"), e(rE, iE, (size_t)dim, thread_cnt, "zlahqr_schur");
@@ -314,17 +321,20 @@ void zlahqr_schur(bool, bool wantZ, int dim, double *rV, double *iV, double *rE,
   Slot zs = wantZ ? Slot(rZ, iZ, nn, thread_cnt, "zlahqr_schur") : Slot(nullptr, nullptr, 0, 1, "zlahqr_schur");
   if (wantZ) z = &zs;
   double *pzr = z ? z->re.data() : zr.data(), *pzi = z ? z->im.data() : zi.data();
-  zlahqr_new(e.re.data(), e.im.data(), v.re.data(), v.im.data(), pzr, pzi, dim, dim * dim, 1, 1);
+  check(veig::slot_zlahqr(dim, slot_batch(block_cnt, thread_cnt), e.re.data(), e.im.data(), v.re.data(), v.im.data(),
+                          pzr, pzi),
+        "zlahqr_schur");
   v.back();
   e.back();
   if (z) z->back();
 }
 
-void ztrevc(double *rT, double *iT, double *, double *, double *rR, double *iR, double *, double *, int dim, int,
-            int thread_cnt) {
+void ztrevc(double *rT, double *iT, double *, double *, double *rR, double *iR, double *, double *, int dim,
+            int block_cnt, int thread_cnt) {
   if (!slot_args(dim, thread_cnt, "ztrevc")) return;
   const size_t nn = (size_t)dim * dim;
   Slot t(rT, iT, nn, thread_cnt, "ztrevc"), r(rR, iR, nn, thread_cnt, "ztrevc");
-  call_ztrevc(dim, 1, 1, t.re.data(), t.im.data(), r.re.data(), r.im.data());
+  check(veig::slot_ztrevc(dim, slot_batch(block_cnt, thread_cnt), t.re.data(), t.im.data(), r.re.data(), r.im.data()),
+        "ztrevc");
   r.back();
 }
