@@ -175,7 +175,7 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_eig_block(E
   const int64_t m = xcd_block();
   if (m >= a.G.nmat) return;  // workgroup-uniform
   const int n = a.G.n;
-  const unsigned top = reduce_load(sm, n, a.G, a.G.mat_base(m), a.rA, a.iA);
+  const unsigned top = reduce_load(sm, n, a.G, a.G.mat_base(m), a.rA, a.iA, [] { return 0u; });
   const int e2 = reduce_block(sm, n, top, nullptr);
   const int lane = threadIdx.x & 63;
   const DenseTile<S::LD> t{sm.H};

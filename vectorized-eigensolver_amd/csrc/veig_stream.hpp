@@ -82,20 +82,21 @@ __device__ __forceinline__ double wave_sum(double x) {
 // the bits above the low word, without the sign: ordered as the magnitudes are,
 // an infinity or a NaN from kNonFinite on
 constexpr unsigned kNonFinite = 0x7ff00000u;
+// the usual range of a largest entry: from 2^-300 to below 2^480
+constexpr unsigned kUsualLow = (1023u - 300u) << 20, kUsualHigh = (1023u + 480u) << 20;
 __device__ __forceinline__ unsigned high_word(double x) {
   return (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32) & 0x7fffffffu;
 }
 __device__ __forceinline__ unsigned high_word(cx<double> x) { return max(high_word(x.re), high_word(x.im)); }
 
 // The power of two that a matrix is divided by before its squares are formed, 0
-// where they fit as it is: with top (the largest high word) between 2^-300 and
-// 2^480 the sums of its squares stay finite, and the square of an entry 2^-150
-// times the largest stays normal.  Exact, so the results are those of the
-// unscaled matrix, scaled.
+// where they fit as it is: with top (the largest high word) in the usual range the
+// sums of its squares stay finite, and the square of an entry 2^-150 times the
+// largest stays normal.  Exact, so the results are those of the unscaled matrix,
+// scaled.
 __device__ __forceinline__ int scale_exponent(unsigned top) {
-  if (top >= kNonFinite) return 0;
-  const int e = (int)(top >> 20) - 1022;  // as frexp's (subnormal: -1022, small enough)
-  return e < -300 || e > 480 ? e : 0;
+  if ((top >= kUsualLow && top < kUsualHigh) || top >= kNonFinite) return 0;
+  return (int)(top >> 20) - 1022;  // as frexp's (subnormal: -1022, small enough)
 }
 // a square below this is taken as zero: an entry below 2^-450, 2^-150 times the
 // largest at most, whose square is on the way to losing its bits
@@ -106,20 +107,25 @@ __device__ __forceinline__ void scale_entries(double2 *h, int count, int thread,
   for (int i = thread; i < count; i += threads) st<double>(h + i, cldexp(ld<double>(h + i), -e));
 }
 
-// the largest high word over the wavefront's count entries
-__device__ __forceinline__ unsigned wave_top(const double2 *h, int count, int lane) {
-  unsigned x = 0;
-  for (int i = lane; i < count; i += 64) x = max(x, high_word(ld<double>(h + i)));
+// The largest high word over the wavefront (exact where it is out of the usual
+// range; in it, some lane's: two votes instead of six exchanges).
+__device__ __forceinline__ unsigned wave_max(unsigned x) {
+  if (__builtin_expect(__any(x >= kUsualLow) && !__any(x >= kUsualHigh), 1)) return kUsualLow;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x = max(x, (unsigned)__shfl_xor((int)x, o));
   return (unsigned)__builtin_amdgcn_readfirstlane((int)x);
 }
 
-// the largest over the workgroup, in every thread (one barrier; words: one LDS
-// word per wavefront)
+// the same over the wavefront's count entries
+__device__ __forceinline__ unsigned wave_top(const double2 *h, int count, int lane) {
+  unsigned x = 0;
+  for (int i = lane; i < count; i += 64) x = max(x, high_word(ld<double>(h + i)));
+  return wave_max(x);
+}
+
+// the same over the workgroup (one barrier; words: one LDS word per wavefront)
 __device__ __forceinline__ unsigned block_max(unsigned x, unsigned *words) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = max(x, (unsigned)__shfl_xor((int)x, o));
+  x = wave_max(x);
   if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = x;
   __syncthreads();
   unsigned m = 0;
@@ -286,14 +292,15 @@ __device__ __forceinline__ int reduce_block(ReduceBlock<CAP, W> &sm, int n, unsi
   return e;
 }
 
-// the tile from memory, zeros outside the matrix (ends at a barrier); returns
-// the largest high word of the matrix and of the thread's `also`
-template <int CAP, int W>
+// the tile from memory, zeros outside the matrix (ends at a barrier); returns the
+// largest high word (block_max).  beside: what else is to be done before the
+// barrier; returns the high word of what it loads.
+template <int CAP, int W, typename F>
 __device__ __forceinline__ unsigned reduce_load(ReduceBlock<CAP, W> &sm, int n, const Geom &G, int64_t base,
-                                                const double *re, const double *im, unsigned also = 0) {
+                                                const double *re, const double *im, F &&beside) {
   constexpr int CH = ReduceBlock<CAP, W>::CH;
   const int r = threadIdx.x % CAP, q = threadIdx.x / CAP;
-  unsigned top = also;
+  unsigned top = 0;
   if (q < W) {
     cx<double> x[CH];
 #pragma unroll
@@ -311,7 +318,7 @@ __device__ __forceinline__ unsigned reduce_load(ReduceBlock<CAP, W> &sm, int n, 
       st<double>(sm.at(r, q * CH + j), x[j]);
     }
   }
-  return block_max(top, sm.words);
+  return block_max(max(top, beside()), sm.words);
 }
 
 // the tile to memory, H times 2^e (the reflectors below its subdiagonal as they are)

@@ -272,7 +272,7 @@ void k_reduce_block_var(VarArgs a, int bin, int part) {
     Gm.nmat = 0;
     Gm.T = 1;
     Gm.n = n;
-    const unsigned top = reduce_load(sm, n, Gm, a.a_off[m], a.rA, a.iA);
+    const unsigned top = reduce_load(sm, n, Gm, a.a_off[m], a.rA, a.iA, [] { return 0u; });
     const int e = reduce_block(sm, n, top, tau);
     reduce_store(sm, n, Gm, a.a_off[m], a.rV, a.iV, e);
     if ((int)threadIdx.x + 1 < n) {
