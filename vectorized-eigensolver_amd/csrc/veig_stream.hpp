@@ -267,28 +267,40 @@ __device__ __forceinline__ void reduce_steps(ReduceBlock<CAP, W> &sm, int n, dou
   }
 }
 
-// (calls: inlined, they cost the usual input's kernels 1 to 3%, in registers and
-// in the order that the rest came out in)
 template <int CAP, int W>
-__device__ __noinline__ void scale_block(ReduceBlock<CAP, W> *sm, int e) {
-  scale_entries(sm->H, (int)(sizeof(sm->H) / sizeof(double2)), threadIdx.x, blockDim.x, e);
+__device__ __forceinline__ void scale_tile(ReduceBlock<CAP, W> &sm, int e) {
+  scale_entries(sm.H, (int)(sizeof(sm.H) / sizeof(double2)), threadIdx.x, blockDim.x, e);
   __syncthreads();
 }
+// the rare forms as calls: inlined, they cost the usual input's kernels 1 to 3% at
+// the capacities from 48 on, in registers and in the order that the rest came out in
 template <int CAP, int W>
-__device__ __noinline__ void reduce_rare(ReduceBlock<CAP, W> *sm, int n, double2 *tau_out) {
+__device__ __noinline__ void scale_call(ReduceBlock<CAP, W> *sm, int e) {
+  scale_tile(*sm, e);
+}
+template <int CAP, int W>
+__device__ __noinline__ void reduce_call(ReduceBlock<CAP, W> *sm, int n, double2 *tau_out) {
   reduce_steps<true>(*sm, n, tau_out);
 }
 
 // top: the largest high word of the input, from reduce_load.  Returns the e of
-// the 2^e that the tile's H is divided by (scale_exponent).
+// the 2^e that the tile's H is divided by (scale_exponent).  (Calls cost a launch
+// about a microsecond, so not at the capacities that small batches take: zgehrd of
+// 64 matrices of order 8 14.6 us with them, 13.7 without.)
 template <int CAP, int W>
 __device__ __forceinline__ int reduce_block(ReduceBlock<CAP, W> &sm, int n, unsigned top, double2 *tau_out) {
+  constexpr bool kCall = CAP > 32;
   const int e = scale_exponent(top);
   if (__builtin_expect(e != 0, 0)) {
-    scale_block(&sm, e);
+    if constexpr (kCall) scale_call(&sm, e);
+    else scale_tile(sm, e);
   }
-  if (__builtin_expect(top >= kNonFinite, 0)) reduce_rare(&sm, n, tau_out);
-  else reduce_steps<false>(sm, n, tau_out);
+  if (__builtin_expect(top >= kNonFinite, 0)) {
+    if constexpr (kCall) reduce_call(&sm, n, tau_out);
+    else reduce_steps<true>(sm, n, tau_out);
+  } else {
+    reduce_steps<false>(sm, n, tau_out);
+  }
   return e;
 }
 
