@@ -18,12 +18,13 @@
  *                (utils.h:37-65); they allocate device memory, copy in, run the
  *                device entry and copy back, like utils.cpp:631-692, and return
  *                after the results are on the host.
- * The kernels of an entry are chosen by order and by number of matrices (batches
- * too small to fill the GPU, orders 4..32, take others; orders 65..93 by
- * how many share a compute unit).  They differ in the order of their operations, so the
- * same matrix in a batch of another size may come out with other last bits, and
- * where rounding decides which eigenvalue deflates first, with E and the columns
- * of V in another order and of another length.  One size gives one result; the
+ * The kernels of an entry are chosen by order and by number of matrices: at orders
+ * 4..32 those of a batch that cannot fill the GPU (up to 1,024 matrices) are other
+ * ones, at 65..93 those of a batch of up to four per compute unit.  They differ in
+ * the order of their operations, so the same matrix in a batch of another size may
+ * come out with other last bits, and where rounding decides which eigenvalue
+ * deflates first, with E and the columns of V in another order and of another
+ * length.  One size gives one result; the
  * per-matrix entries of veig_compat.hpp follow the batch they are told of.
  * Every function returns a veig_status; veig_last_error() describes the last
  * failure of the calling thread.  Sizes are 64-bit (the reference's 32-bit
@@ -75,7 +76,7 @@ const char *veig_version(void);
  * info (may be NULL): per matrix, the number of eigenvalues accepted after
  * `itmax` sweeps without a negligible subdiagonal (the reference caps at 30,
  * Toolbox.hpp:808, and reports nothing; itmax <= 0 selects 30).
- * A, E and V are separate arrays: above order 8 the call passes the
+ * A, E and V are separate arrays: from order 8 on the call passes the
  * Hessenberg reduction's compact form between its kernels through V and E,
  * which then receive the results.
  * ------------------------------------------------------------------------- */
@@ -113,7 +114,8 @@ int veig_zgeev_mixed(int64_t dim, int64_t block_cnt, int64_t thread_cnt, const d
 
 /* ---------------------------------------------------------------------------
  * Batches of different orders.  No counterpart in the reference (its batches
- * are equal-size, utils.cpp:578); the per-matrix arithmetic is veig_zgeev's.
+ * are equal-size, utils.cpp:578); the per-matrix arithmetic is that of veig_zgeev
+ * on a large batch.
  * Matrix m (order dims[m], 0 <= dims[m] <= 32) is column-major with leading
  * dimension dims[m] at offset a_off[m] of the rA/iA planes; its eigenvectors
  * go to the same offsets of rV/iV and its eigenvalues to e_off[m] of rE/iE.

@@ -45,8 +45,10 @@ enum { ST_GEHRD = 0, ST_HESS = 1, ST_UNGHR = 2, ST_LAHQR = 3, ST_TREVC = 4 };
 // (65,536 matrices, lane groups -> workgroups: hessenberg of order 17 2.58 ->
 // 2.25 ms, 24 4.42 -> 3.01, 32 7.03 -> 4.00; ztrevc 1.11 -> 0.95, 1.92 -> 1.49,
 // 2.88 -> 2.27; at order 16 they lose, 0.65 -> 0.71 and 0.33 -> 0.73).  Below
-// it the reduction does up to four matrices per CU (order 16 x 1,024: 68 ->
-// 44 us), the QR iteration up to one (few_matrices).  batch: the matrices of
+// it the reduction does up to four matrices per CU, the QR iteration up to one
+// (few_matrices).  zgehrd of 64 / 1,024 matrices, us: order 8 18.1 -> 13.8, 18.4
+// -> 16; 12 30.3 -> 18.9, 30.9 -> 21.4; 16 46.0 -> 23.8, 47.2 -> 26.8; zunghr of
+// order 8 9.0 -> 8.8, 9.0 -> 9.2, 16 17.5 -> 11.8, 18.0 -> 13.3.  batch: the matrices of
 // the batch, or of the one that a single matrix is taken out of (veig_slot.hpp).
 bool per_workgroup(int mode, int n, int64_t batch) {
   if (n > 32) return true;
@@ -230,6 +232,9 @@ __global__ void k_layout(int dir, Geom G, const double *in, double *out, int64_t
 
 int launch_stage(const StageArgs &a, hipStream_t s) {
   const int nb = nb_for(a.G.n);
+  // k_stage<32> is the QR iteration whatever the mode (see per_workgroup)
+  if (nb > 32 || (nb > 16 && a.mode != ST_LAHQR))
+    return fail(VEIG_ERR_UNSUPPORTED, "this stage runs one matrix per workgroup at this order");
   const int mpw = 64 / nb;
   const int64_t grid = (a.G.nmat + mpw - 1) / mpw;
   if (grid > INT32_MAX) return fail(VEIG_ERR_INVALID, "batch too large for one launch");

@@ -8,8 +8,8 @@
 //                      (reduce_block); for the fused path its compact form
 //                      goes to the V and E planes, which serve as workspace;
 //                      for the stages also Q (hessenberg, zunghr).
-//   k_schur<SL, NT>    wavefront 0 runs the QR iteration on the banded tile
-//                      (lahqr_stream), the others hold the Schur vectors in
+//   k_schur<SL, NT>    one wavefront (chain_wave) runs the QR iteration on the
+//                      banded tile (lahqr_stream), the others hold the Schur vectors in
 //                      registers, NT lanes per row, and replay the recorded
 //                      sweeps (SchurRows); then the eigenvector solve and
 //                      V = Z X on the matrix cores.
@@ -24,8 +24,9 @@
 // order: 40 KB at n = 64 (four matrices per CU), 71 KB at n = 88 (two).
 //
 // Measured, whole passes (in brackets the kernels these replaced, whose bulge
-// chase went through LDS): order 64 x 65,536 181 ms (371), order 79 x 3,328
-// 34 ms (233: a workgroup barrier per half step and Z in global memory), the
+// chase went through LDS): order 64 x 65,536 182 ms (371; reduction 25,
+// k_schur 153 in a trace), order 79 x 3,328 31.6 ms (233: a workgroup barrier per
+// half step and Z in global memory; reduction 3.6, k_schur 27.9), the
 // stages hessenberg + zlahqr + ztrevc at order 40 x 2,048 3.1 ms (21).  What
 // bounds order 64 is instruction issue, the chain wavefront's (7,700 steps of
 // about 88 instructions and 230 sweeps of about 480 more per matrix) and,

@@ -162,8 +162,8 @@ __global__ __launch_bounds__(64) void k_eig(EigArgs a) {
 }
 
 // Orders 33..64 (and few matrices of a smaller order), eigenvalues only: the reduction by the whole workgroup on a
-// dense tile, then the iteration by its first wavefront in the same tile
-// (lahqr_stream; the others are done).  Order 48 x 16,384: 20.2 ms, against
+// dense tile, then the iteration by one of its wavefronts (chain_wave) in the
+// same tile (lahqr_stream; the others are done).  Order 48 x 16,384: 20.3 ms, against
 // 60.7 ms for one wavefront doing both on a 66 KB tile; at 41 KB four
 // workgroups share a CU, one chain per SIMD, and the chain's issue rate bounds
 // them (see lahqr_stream).
