@@ -82,3 +82,28 @@ def test_subdiagonal_far_below_the_rest(gpu, n):
     E, V, info = gpu_eig(A, 1)
     assert np.all(info == 0) and np.all(np.isfinite(V))
     assert np.all(H.backward_error(A, E, V) <= 64 * n * np.finfo(float).eps)
+
+
+@pytest.mark.parametrize("k", [-960, -700])
+@pytest.mark.parametrize("route", ["batch", "uneven", "mixed"])
+@pytest.mark.parametrize("n", [12, 16, 20, 24, 27, 28, 32])
+def test_lane_groups_report_what_they_lose(gpu, n, route, k):
+    # the QR iteration on lane groups does not scale: such a matrix is reported
+    # (info) or undefined, never returned as converged and wrong
+    A = np.tile(H.gaussian(3, n, 9970 + n) * 2.0 ** k, (101, 1, 1))
+    if route == "uneven":
+        from test_gpu_varsize import fetch
+        vb = veig.VarBatch([n] * len(A))
+        vb.rA.copy_(torch.from_numpy(np.ascontiguousarray(np.swapaxes(A, 1, 2)).reshape(-1).real.copy()))
+        vb.iA.copy_(torch.from_numpy(np.ascontiguousarray(np.swapaxes(A, 1, 2)).reshape(-1).imag.copy()))
+        vb.run()
+        torch.cuda.synchronize()
+        out = fetch(vb, [n] * len(A))
+        E, V, info = np.stack([o[0] for o in out]), np.stack([o[1] for o in out]), vb.info.cpu().numpy()
+    else:
+        E, V, info = gpu_eig(A, 1, precision="mixed" if route == "mixed" else "fp64")[:3]
+    silent = (info == 0) & np.all(np.isfinite(E), axis=1)
+    if np.any(silent):
+        want, _, _ = H.oracle_eig(A[silent] * 2.0 ** -k, 1)
+        _, err = H.match_eigenvalues(want, E[silent] * 2.0 ** -k)
+        assert np.all(err <= 1e-9 * np.linalg.norm(A[silent] * 2.0 ** -k, axis=(1, 2)))

@@ -69,7 +69,7 @@ __device__ __forceinline__ bool block_matrix(const BigArgs &a, int64_t &m) {
 // ---------------------------------------------------------------------------
 // reduction
 // ---------------------------------------------------------------------------
-enum { RD_FUSED = 0, RD_GEHRD = 1, RD_HESS = 2, RD_UNGHR = 3 };
+enum { RD_FUSED = 0, RD_GEHRD = 1, RD_HESS = 2, RD_UNGHR = 3, RD_BANDED = 4 };  // (banded: for k_qr_band)
 
 // (at most three wavefronts per SIMD at capacity 24: four, which zunghr's registers
 // allow, took 1.23 ms instead of 0.75 at 65,536 matrices of order 24 in tiles of 64,
@@ -96,8 +96,8 @@ void k_reduce(BigArgs a) {
     });
   } else {
     top = reduce_load(sm, n, a.G, base, a.rA, a.iA, [] { return 0u; });
-    const int e = reduce_block(sm, n, top, tau);
-    const bool fused = MODE == RD_FUSED;
+    const int e = reduce_block<MODE != RD_BANDED>(sm, n, top, tau);
+    const bool fused = MODE == RD_FUSED || MODE == RD_BANDED;
     reduce_store(sm, n, a.G, base, fused ? a.rB : a.rA, fused ? a.iB : a.iA, e);
     if (a.rE && tid + 1 < n) {
       const cx<double> t = ld<double>(tau + tid);
@@ -340,7 +340,8 @@ int launch_big(int mode, const Geom &G, double *rA, double *iA, double *rB, doub
     case BIG_FUSED:
       VEIG_TRY(reduce_for<RD_FUSED>(a, s));
       return schur_for<SC_FUSED>(a, s, batch);
-    case BIG_REDUCE: return reduce_for<RD_FUSED>(a, s);
+    case BIG_REDUCE:  // orders 17..32
+      return G.n <= 24 ? launch_reduce<24, 2, RD_BANDED>(a, s) : launch_reduce<32, 4, RD_BANDED>(a, s);
     case BIG_GEHRD: return reduce_for<RD_GEHRD>(a, s);
     case BIG_HESS: return reduce_for<RD_HESS>(a, s);
     case BIG_UNGHR: return reduce_for<RD_UNGHR>(a, s);

@@ -176,7 +176,7 @@ __global__ __launch_bounds__((ReduceBlock<CAP, W>::kThreads)) void k_eig_block(E
   if (m >= a.G.nmat) return;  // workgroup-uniform
   const int n = a.G.n;
   const unsigned top = reduce_load(sm, n, a.G, a.G.mat_base(m), a.rA, a.iA, [] { return 0u; });
-  const int e2 = reduce_block(sm, n, top, nullptr);
+  const int e2 = reduce_block<true>(sm, n, top, nullptr);
   const int lane = threadIdx.x & 63;
   const DenseTile<S::LD> t{sm.H};
   auto &rec = *reinterpret_cast<SweepScratch<CAP> *>(sm.part);  // free now

@@ -164,7 +164,9 @@ struct ReduceBlock {
   __device__ __forceinline__ double2 *v(int c) { return H + c * LD + CAP; }  // the reflector's entry c
 };
 
-template <bool kRare, int CAP, int W>
+// kTiny: columns whose square is below kTinySquare are taken as zero (in a tile
+// that has been scaled).
+template <bool kRare, bool kTiny, int CAP, int W>
 __device__ __forceinline__ void reduce_steps(ReduceBlock<CAP, W> &sm, int n, double2 *tau_out) {
   using R = double;
   constexpr int CH = ReduceBlock<CAP, W>::CH;
@@ -181,7 +183,7 @@ __device__ __forceinline__ void reduce_steps(ReduceBlock<CAP, W> &sm, int n, dou
     cx<R> tau = mk<R>(0, 0), scal = mk<R>(0, 0);
     R beta = alpha.re;
     const R nrm2 = abs2(alpha) + xnorm2;
-    if (!(xnorm2 == 0.0 && alpha.im == 0.0) && !(nrm2 < kTinySquare)) {
+    if (!(xnorm2 == 0.0 && alpha.im == 0.0) && !(kTiny && nrm2 < kTinySquare)) {
       const R nrm = fsqrt(nrm2);
       beta = alpha.re >= 0.0 ? -nrm : nrm;
       const R ib = frcp(beta);
@@ -278,28 +280,31 @@ template <int CAP, int W>
 __device__ __noinline__ void scale_call(ReduceBlock<CAP, W> *sm, int e) {
   scale_tile(*sm, e);
 }
-template <int CAP, int W>
+template <bool kScale, int CAP, int W>
 __device__ __noinline__ void reduce_call(ReduceBlock<CAP, W> *sm, int n, double2 *tau_out) {
-  reduce_steps<true>(*sm, n, tau_out);
+  reduce_steps<true, kScale>(*sm, n, tau_out);
 }
 
 // top: the largest high word of the input, from reduce_load.  Returns the e of
 // the 2^e that the tile's H is divided by (scale_exponent).  (Calls cost a launch
 // about a microsecond, so not at the capacities that small batches take: zgehrd of
 // 64 matrices of order 8 14.6 us with them, 13.7 without.)
-template <int CAP, int W>
+// kScale = false, for the QR iteration on lane groups, which does not scale: a
+// matrix out of the range stays undefined, as there, where its H would come out of
+// an iteration without squares as converged and wrong.
+template <bool kScale, int CAP, int W>
 __device__ __forceinline__ int reduce_block(ReduceBlock<CAP, W> &sm, int n, unsigned top, double2 *tau_out) {
   constexpr bool kCall = CAP > 32;
-  const int e = scale_exponent(top);
+  const int e = kScale ? scale_exponent(top) : 0;
   if (__builtin_expect(e != 0, 0)) {
     if constexpr (kCall) scale_call(&sm, e);
     else scale_tile(sm, e);
   }
   if (__builtin_expect(top >= kNonFinite, 0)) {
-    if constexpr (kCall) reduce_call(&sm, n, tau_out);
-    else reduce_steps<true>(sm, n, tau_out);
+    if constexpr (kCall) reduce_call<kScale>(&sm, n, tau_out);
+    else reduce_steps<true, kScale>(sm, n, tau_out);
   } else {
-    reduce_steps<false>(sm, n, tau_out);
+    reduce_steps<false, kScale>(sm, n, tau_out);
   }
   return e;
 }

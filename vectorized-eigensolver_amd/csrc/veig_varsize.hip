@@ -273,8 +273,8 @@ void k_reduce_block_var(VarArgs a, int bin, int part) {
     Gm.T = 1;
     Gm.n = n;
     const unsigned top = reduce_load(sm, n, Gm, a.a_off[m], a.rA, a.iA, [] { return 0u; });
-    const int e = reduce_block(sm, n, top, tau);
-    reduce_store(sm, n, Gm, a.a_off[m], a.rV, a.iV, e);
+    (void)reduce_block<false>(sm, n, top, tau);
+    reduce_store(sm, n, Gm, a.a_off[m], a.rV, a.iV, 0);
     if ((int)threadIdx.x + 1 < n) {
       const cx<double> t = ld<double>(tau + threadIdx.x);
       a.rE[a.e_off[m] + threadIdx.x] = t.re;
